@@ -639,6 +639,31 @@ int tmac_silu_bwd(const void* d_dh, const void* d_z, void* d_dz, int64_t n, int 
 int tmac_mse_grad(const void* d_y, const void* d_v, void* d_dy, int64_t n, float coef, int dtype,
                   void* stream);
 
+/* ------------------------------------------------------------------------
+ * Dense projections: nn.Linear without bias on 16-bit inputs (fp32
+ * accumulation), the qkv and output projections of the attention modules
+ * (attn/windowed_attention.py:295-299, :331; attn/block_sparse_attention.py:222-223, :340).
+ *
+ * W is [N, K] (out, in) row-major as nn.Linear stores it; N and K are multiples
+ * of 64; every pointer is 16-byte aligned and every pitch a multiple of 8, at
+ * most 2^22 elements. dtype: TMAC_BF16 or TMAC_F16.
+ * ------------------------------------------------------------------------ */
+
+/* Y[M, N] = X[M, K] · Wᵀ. */
+int tmac_linear_fwd(const void* d_X, int64_t ldx, const void* d_W, int64_t ldw, void* d_Y,
+                    int64_t ldy, int M, int N, int K, int dtype, void* stream);
+
+/* dX[M, K] = dY[M, N] · W. */
+int tmac_linear_dx(const void* d_dY, int64_t lddy, const void* d_W, int64_t ldw, void* d_dX,
+                   int64_t lddx, int M, int N, int K, int dtype, void* stream);
+
+/* dW[N, K] = dYᵀ · X, contiguous, in dtype. The sums over row ranges are fp32 and
+ * added in a fixed order (deterministic for given sizes); they go to d_ws, of
+ * tmac_linear_wgrad_workspace bytes (0: no workspace needed, d_ws may be NULL). */
+int tmac_linear_wgrad_workspace(int M, int N, int K, size_t* ws_bytes);
+int tmac_linear_wgrad(const void* d_dY, int64_t lddy, const void* d_X, int64_t ldx, void* d_dW,
+                      void* d_ws, size_t ws_bytes, int M, int N, int K, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,119 @@
+"""Dense projections (kernels/linear.py): the HIP kernels against fp64 products of the same inputs, at
+the edges of their tiles, and the calls that stay with torch."""
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from titans_core.kernels import _lib
+from titans_core.kernels import linear as ln
+
+HALF = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}  # unit roundoff of the stored result
+
+
+def _close(got, a, b):
+    """got = a @ b up to the rounding of the stored value and of fp32 sums in any order: (K + 1) 2^-24
+    times the sum of magnitudes bounds them; fp16 results below its normal range add 2^-25."""
+    ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    bound = HALF[got.dtype] * ref.abs() + (a.shape[1] + 1) * 2.0 ** -24 * mag * (1 + HALF[got.dtype]) + 2.0 ** -24
+    err = (got.double() - ref).abs()
+    assert torch.all(err <= bound), f"max excess {(err - bound).max().item():.3g}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (31, 64, 128), (64, 128, 64), (191, 192, 320),
+                                   (193, 320, 192), (385, 256, 640), (515, 576, 128), (1000, 640, 192)])
+def test_kernels_at_tile_edges(dev, M, N, K, dtype):
+    g = torch.Generator().manual_seed(M + N + K)
+    wide = torch.randn(M, K + 72, generator=g).to(dev, dtype)
+    x = wide[:, 8:K + 8]  # a column slice: pitch K + 72, 16-byte aligned
+    w = torch.randn(N, K, generator=g).to(dev, dtype)
+    gy = torch.randn(M, N, generator=g).to(dev, dtype)
+    _close(ln._fwd(x, w), x, w.t())
+    _close(ln._dx(gy, w), gy, w)
+    _close(ln._wgrad(gy, x), gy.t(), x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4099, 64, 64), (9001, 192, 640), (9001, 640, 192)])
+def test_wgrad_split_over_rows(dev, M, N, K):
+    nb = ctypes.c_size_t(0)
+    assert _lib.lib().tmac_linear_wgrad_workspace(M, N, K, ctypes.byref(nb)) == 0 and nb.value > 0
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(dev, torch.bfloat16)
+    gy = torch.randn(M, N, generator=g).to(dev, torch.bfloat16)
+    a = ln._wgrad(gy, x)
+    _close(a, gy.t(), x)
+    assert torch.equal(a, ln._wgrad(gy, x))
+
+
+@pytest.mark.gpu
+def test_rows_past_the_end_do_not_leak(dev):
+    """Infinities in the last row reach only what that row contributes to."""
+    x = torch.ones(200, 64, device=dev, dtype=torch.bfloat16)
+    x[-1] = float("inf")
+    w = torch.ones(64, 64, device=dev, dtype=torch.bfloat16)
+    y = ln._fwd(x, w)
+    assert torch.all(y[:-1] == 64) and torch.all(torch.isinf(y[-1]))
+    gy = torch.ones(200, 64, device=dev, dtype=torch.bfloat16)
+    gy[-1] = 0
+    x[-1] = 3
+    assert torch.all(ln._wgrad(gy, x) == 199)
+
+
+@pytest.mark.gpu
+def test_projection_gradients_and_modes(dev):
+    g = torch.Generator().manual_seed(3)
+    p = ln.Projection(192, 640).to(dev, torch.bfloat16)
+    x = torch.randn(10, 1201, 192, generator=g).to(dev, torch.bfloat16).requires_grad_()
+    gy = torch.randn(10, 1201, 640, generator=g).to(dev, torch.bfloat16)
+    y = p(x)
+    _close(y.detach().reshape(-1, 640), x.detach().reshape(-1, 192), p.weight.detach().t())
+    y.backward(gy)
+    _close(x.grad.reshape(-1, 192), gy.reshape(-1, 640), p.weight.detach())
+    _close(p.weight.grad, gy.reshape(-1, 640).t(), x.detach().reshape(-1, 192))
+    # an expanded gradient (stride 0) and a hook on the saved tensors
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(1) or t, lambda t: t):
+        y = p(x)
+    assert seen
+    x.grad = p.weight.grad = None
+    y.sum().backward()
+    ones = torch.ones(12010, 640, device=dev, dtype=torch.bfloat16)
+    _close(x.grad.reshape(-1, 192), ones, p.weight.detach())
+    # double backward, functorch and forward-mode AD stay with torch's products
+    (gx,) = torch.autograd.grad(p(x).float().pow(2).sum(), x, create_graph=True)
+    gx.float().sum().backward()
+    out = torch.func.vmap(p)(x.detach())
+    assert out.shape == (10, 1201, 640)
+    with torch.autograd.forward_ad.dual_level():
+        d = torch.autograd.forward_ad.make_dual(x.detach(), torch.ones_like(x))
+        assert torch.autograd.forward_ad.unpack_dual(p(d)).tangent is not None
+    # autocast: fp32 module, 16-bit product
+    q = ln.Projection(192, 640).to(dev)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = q(x.detach().float())
+    assert y.dtype == torch.bfloat16
+    _close(y.detach().reshape(-1, 640), x.detach().reshape(-1, 192), q.weight.detach().bfloat16().t())
+
+
+def test_projection_on_the_cpu_is_nn_linear():
+    p = ln.Projection(64, 128)
+    x = torch.randn(3, 5, 64, requires_grad=True)
+    assert isinstance(p, torch.nn.Linear) and p.bias is None
+    assert torch.equal(p(x), F.linear(x, p.weight))
+
+
+def test_argument_errors():
+    L, p = _lib.lib(), 4096  # an aligned address; nothing is launched
+    nb = ctypes.c_size_t(0)
+    assert L.tmac_linear_fwd(0, 64, p, 64, p, 64, 8, 64, 64, _lib.BF16, None) == -1
+    assert L.tmac_linear_fwd(p, 64, p, 64, p, 64, 8, 63, 64, _lib.BF16, None) == -2
+    assert L.tmac_linear_fwd(p, 32, p, 64, p, 64, 8, 64, 64, _lib.BF16, None) == -2
+    assert L.tmac_linear_fwd(p, 64, p, 64, p, 64, 8, 64, 64, _lib.F32, None) == -4
+    assert L.tmac_linear_dx(p + 2, 64, p, 64, p, 64, 8, 64, 64, _lib.BF16, None) == -5
+    assert L.tmac_linear_dx(p, 1 << 23, p, 64, p, 64, 8, 64, 64, _lib.BF16, None) == -2
+    assert L.tmac_linear_wgrad_workspace(0, 64, 64, ctypes.byref(nb)) == -2
+    assert L.tmac_linear_wgrad(p, 64, p, 64, p, None, 0, 1 << 16, 64, 64, _lib.BF16, None) == -6

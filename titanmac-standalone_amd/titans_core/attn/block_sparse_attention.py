@@ -33,6 +33,7 @@ import torch
 import torch.nn as nn
 
 from ..kernels.conv import causal_dwconv
+from ..kernels.linear import Projection
 from ..kernels.window_attn import windowed_attention
 
 
@@ -54,12 +55,12 @@ class BlockSparseAttention(nn.Module):
         self.dropout_p = dropout
         self.causal = causal
         self.use_conv = use_conv
-        self.qkv_proj = nn.Linear(d_model, 3 * d_model, bias=False)
+        self.qkv_proj = Projection(d_model, 3 * d_model)
         if use_conv:
             mk = lambda: nn.Conv1d(d_model, d_model, kernel_size=conv_kernel,  # noqa: E731
                                    padding=conv_kernel - 1, groups=d_model, bias=False)
             self.conv_q, self.conv_k, self.conv_v = mk(), mk(), mk()
-        self.out_proj = nn.Linear(d_model, d_model, bias=False)
+        self.out_proj = Projection(d_model, d_model)
         self.dropout = nn.Dropout(dropout) if dropout > 0 else nn.Identity()
         self.scale = 1.0 / math.sqrt(self.d_head)
 

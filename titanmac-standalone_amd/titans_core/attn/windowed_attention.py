@@ -21,6 +21,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
+from ..kernels.linear import Projection
 from ..kernels.window_attn import windowed_attention
 
 
@@ -98,8 +99,8 @@ class WindowedAttention(nn.Module):
             self.dropout_p = config.attention_dropout
         assert self.d_model == self.n_heads * self.d_head, \
             f"d_model ({self.d_model}) must equal n_heads ({self.n_heads}) * d_head ({self.d_head})"
-        self.qkv_proj = nn.Linear(self.d_model, 3 * self.d_model, bias=False)
-        self.out_proj = nn.Linear(self.d_model, self.d_model, bias=False)
+        self.qkv_proj = Projection(self.d_model, 3 * self.d_model)
+        self.out_proj = Projection(self.d_model, self.d_model)
         self.dropout = nn.Dropout(self.dropout_p) if self.dropout_p > 0 else nn.Identity()
         self._mask_cache = {}
 

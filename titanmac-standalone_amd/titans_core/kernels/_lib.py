@@ -82,6 +82,10 @@ SIGNATURES = {
                           _vp, _vp, _vp, _i, _i, _vp, _vp],
     "tmac_wattn_mask_lists": [_vp, _i, _vp],
     "tmac_wattn_mask_grad_reduce": [_vp, _i, _i, _i, _i, _i, _vp, _vp],
+    "tmac_linear_fwd": [_vp, _i64, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
+    "tmac_linear_dx": [_vp, _i64, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
+    "tmac_linear_wgrad_workspace": [_i, _i, _i, ctypes.POINTER(_sz)],
+    "tmac_linear_wgrad": [_vp, _i64, _vp, _i64, _vp, _vp, _sz, _i, _i, _i, _i, _vp],
     "tmac_dwconv_causal": [_vp, _i64, _vp, _vp, _i64, _i, _i, _i, _i, _i, _vp],
     "tmac_dwconv_causal_bwd_workspace": [_i, _i, _i, _i, ctypes.POINTER(_sz)],
     "tmac_dwconv_causal_bwd": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _sz, _i, _i, _i, _i,
@@ -189,6 +193,17 @@ def direct_call(*tensors: torch.Tensor | None) -> bool:
         if type(t) not in _PLAIN or (grad and t.requires_grad):
             return False
     return True
+
+
+def eager_native(*tensors: torch.Tensor | None) -> bool:
+    """Whether an op may record its autograd node with a plain autograd.Function and run its kernels
+    directly: eager mode, plain tensors, and nothing that rewrites, traces or intercepts torch calls
+    (torch.compile, functorch transforms, forward-mode AD, function or dispatch modes)."""
+    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()):
+        return False
+    return all(t is None or type(t) in _PLAIN for t in tensors)
 
 
 def require_device(*tensors: torch.Tensor, what: str) -> torch.device:

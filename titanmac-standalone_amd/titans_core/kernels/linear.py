@@ -1,0 +1,170 @@
+"""Bias-free dense projections on the GPU (HIP kernels for gfx950).
+
+The attention modules' qkv and output projections are ``nn.Linear(..., bias=False)``
+(attn/windowed_attention.py:229-230, attn/block_sparse_attention.py:84, :101). ``projection``
+computes ``F.linear(x, weight)``: 16-bit GPU inputs run the MFMA kernels of
+``csrc/linear_kernels.hip`` (forward, input and weight gradient), everything else torch's own.
+``Projection`` is an ``nn.Linear`` whose forward calls it.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from . import _lib
+
+_HALF = (torch.bfloat16, torch.float16)
+_MAX_PITCH = 1 << 22  # the kernels address a tile's rows with 32-bit offsets
+_MAX_WEIGHT, _MAX_ROWS = 1 << 30, 1 << 30
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """t as [M, features] rows the kernels can read: unit column stride, a row pitch of a multiple of
+    8 elements, a 16-byte aligned start (copied if it has not got that)."""
+    t2 = t.reshape(-1, t.shape[-1])
+    if (t2.stride(1) != 1 or t2.stride(0) < t2.shape[1] or t2.stride(0) % 8
+            or t2.stride(0) > _MAX_PITCH or t2.data_ptr() % 16):
+        t2 = t2.clone(memory_format=torch.contiguous_format)
+    return t2
+
+
+def _fwd(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    (M, K), N = x2.shape, w.shape[0]
+    y = torch.empty((M, N), dtype=x2.dtype, device=x2.device)
+    with _lib.device_guard(x2.device):
+        rc = _lib.lib().tmac_linear_fwd(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
+                                        M, N, K, _lib.dtype_code(x2.dtype), _lib.stream_ptr(x2.device))
+    _lib.check(rc, "tmac_linear_fwd")
+    return y
+
+
+def _dx(g2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    (M, N), K = g2.shape, w.shape[1]
+    dx = torch.empty((M, K), dtype=g2.dtype, device=g2.device)
+    with _lib.device_guard(g2.device):
+        rc = _lib.lib().tmac_linear_dx(g2.data_ptr(), g2.stride(0), w.data_ptr(), w.stride(0), dx.data_ptr(), K,
+                                       M, N, K, _lib.dtype_code(g2.dtype), _lib.stream_ptr(g2.device))
+    _lib.check(rc, "tmac_linear_dx")
+    return dx
+
+
+def _wgrad(g2: torch.Tensor, x2: torch.Tensor) -> torch.Tensor:
+    (M, N), K = g2.shape, x2.shape[1]
+    L = _lib.lib()
+    nb = ctypes.c_size_t(0)
+    _lib.check(L.tmac_linear_wgrad_workspace(M, N, K, ctypes.byref(nb)), "tmac_linear_wgrad_workspace")
+    ws = torch.empty(nb.value, dtype=torch.uint8, device=g2.device)
+    dw = torch.empty((N, K), dtype=g2.dtype, device=g2.device)
+    with _lib.device_guard(g2.device):
+        rc = L.tmac_linear_wgrad(g2.data_ptr(), g2.stride(0), x2.data_ptr(), x2.stride(0), dw.data_ptr(),
+                                 ws.data_ptr(), nb.value, M, N, K, _lib.dtype_code(g2.dtype),
+                                 _lib.stream_ptr(g2.device))
+    _lib.check(rc, "tmac_linear_wgrad")
+    return dw
+
+
+# Where each kernel replaces the library's GEMM: where it measured faster (us, this kernel / library,
+# GPU time of [M, K] x [N, K] in bf16; `tiles` counts its 192 x 128 output tiles). A tile walks its
+# reduction in order, so few tiles or long walks leave the chip idle, and at K >= 1024 the library's
+# larger tiles read less through LDS.
+
+def _tiles(rows: int, cols: int) -> int:
+    return -(-rows // 192) * -(-cols // 128)
+
+
+def _fwd_applies(M: int, N: int, K: int) -> bool:
+    """(2240, 640, 1920), 180 tiles: 12.1 / 15.0; (17920, 640, 1920): 54 / 80; (17920, 640, 640): 19 / 36;
+    below: (1100, 640, 1920), 90 tiles: 10.6 / 9.3; (9000, 1024, 3072): 60 / 51."""
+    return K <= 768 and _tiles(M, N) >= 150
+
+
+def _dx_applies(M: int, N: int, K: int) -> bool:
+    """(17920, 640, 1920), 470 tiles: 43 / 61; (9000, 1024, 3072), 376: 55 / 68; (4480, 640, 640), 120:
+    11.3 / 13.5; below: (4480, 640, 1920), 120: 26.2 / 25.2; (2240, 640, 640), 60: 10.7 / 8.4."""
+    return _tiles(M, K) >= (100 if N <= 1024 else 256)
+
+
+def _wgrad_applies(M: int) -> bool:
+    """The library gives these products few tiles and no split over M: (17920, 640, 1920): 59 / 141;
+    (17920, 640, 640): 28 / 102; (1100, 640, 640): 12.8 / 13.3; below: (256, 640, 640): 7.4 / 6.1."""
+    return M >= 512
+
+
+def _forward(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    N, K = weight.shape
+    if not _fwd_applies(x.numel() // K, N, K):
+        return F.linear(x, weight)
+    return _fwd(_rows(x), _rows(weight)).view(*x.shape[:-1], N)
+
+
+class _Projection(torch.autograd.Function):
+    """F.linear(x, weight) with its gradients on the kernels. A backward that is itself differentiated
+    (create_graph) uses torch's products, as nn.Linear's own double backward does."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        ctx.save_for_backward(x, weight)
+        return _forward(x, weight)
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, weight = ctx.saved_tensors
+        gx = gw = None
+        if torch.is_grad_enabled() or not _lib.eager_native(gy, x, weight):
+            if ctx.needs_input_grad[0]:
+                gx = gy @ weight
+            if ctx.needs_input_grad[1]:
+                gw = gy.reshape(-1, gy.shape[-1]).t() @ x.reshape(-1, x.shape[-1])
+            return gx, gw
+        g2 = _rows(gy)
+        M, N = g2.shape
+        if ctx.needs_input_grad[0]:
+            gx = _dx(g2, _rows(weight)) if _dx_applies(M, N, weight.shape[1]) else g2 @ weight
+            gx = gx.view(x.shape)
+        if ctx.needs_input_grad[1]:
+            x2 = x.reshape(-1, x.shape[-1])
+            gw = _wgrad(g2, _rows(x2)) if _wgrad_applies(M) else g2.t() @ x2
+        return gx, gw
+
+
+def projection(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, weight): [..., K] x [N, K] -> [..., N]. The kernels take bfloat16 and float16 (inside
+    torch.autocast the inputs are cast to its dtype, as F.linear's are) with N and K multiples of 64."""
+    ac = torch.is_autocast_enabled("cuda")
+    if not (ac or x.dtype in _HALF) or not (x.is_cuda and weight.is_cuda and _lib.eager_native(x, weight)):
+        return F.linear(x, weight)
+    if ac:
+        dt = torch.get_autocast_dtype("cuda")
+        if dt in _HALF and x.dtype in (torch.float32, *_HALF) and weight.dtype in (torch.float32, *_HALF):
+            x, weight = x.to(dt), weight.to(dt)
+            with torch.autocast("cuda", enabled=False):
+                return _projection(x, weight)
+        return F.linear(x, weight)
+    return _projection(x, weight)
+
+
+def _projection(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """projection outside autocast, of plain GPU tensors."""
+    if (x.dtype not in _HALF or weight.dtype != x.dtype or weight.device != x.device or weight.dim() != 2
+            or x.dim() < 1 or x.shape[-1] != weight.shape[1] or x.numel() == 0):
+        return F.linear(x, weight)
+    (N, K), M = weight.shape, x.numel() // x.shape[-1]
+    if (N == 0 or N % 64 or K % 64 or max(N, K) > _MAX_PITCH or N * K > _MAX_WEIGHT or M > _MAX_ROWS
+            or not (_wgrad_applies(M) or _fwd_applies(M, N, K))):
+        return F.linear(x, weight)
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+        return _Projection.apply(x, weight)
+    return _forward(x, weight)
+
+
+class Projection(nn.Linear):
+    """nn.Linear(in_features, out_features, bias=False) on ``projection``."""
+
+    def __init__(self, in_features: int, out_features: int):
+        super().__init__(in_features, out_features, bias=False)
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return projection(x, self.weight)
