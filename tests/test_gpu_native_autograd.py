@@ -1,0 +1,91 @@
+"""Training calls record a plain autograd.Function in eager mode and the registered torch.library op
+where calls are traced, transformed or intercepted. Both routes: the same bits, results and gradients."""
+import pytest
+import torch
+
+from titans_core.kernels import _lib
+from titans_core.kernels import block_ell as kb
+from titans_core.kernels.conv import causal_dwconv
+from titans_core.kernels.norm import rms_norm
+from titans_core.kernels.window_attn import windowed_attention
+
+
+def _block_ell(activation):
+    pat = kb.BlockELLPattern.sample(1, 3, 5, 2)
+    return (lambda x, v, b: kb.block_ell_mm(x, v, pat, b, activation)), [(90, 192), (3, 2, 64, 64), (320,)]
+
+
+def _attention(**kw):
+    return (lambda q, k, v: windowed_attention(q, k, v, 40, 4, **kw)), [(2, 2, 100, 64)] * 3
+
+
+CASES = {
+    "norm": (lambda x, s: rms_norm(x, s), [(70, 128), (128,)]),
+    "conv": (causal_dwconv, [(2, 75, 128), (128, 4)]),
+    "linear": _block_ell(None),
+    "linear_gelu": _block_ell("gelu"),
+    "attention": _attention(),
+    "attention_dropout": _attention(dropout_p=0.25, seed=11),
+}
+
+
+def _grads(fn, shapes, dtype, dev):
+    g = torch.Generator().manual_seed(5)
+    xs = [(torch.randn(*s, generator=g) * 0.3).to(dev, dtype).requires_grad_() for s in shapes]
+    y = fn(*xs)
+    y.backward(torch.randn(y.shape, generator=g).to(dev, dtype))
+    return [y.detach()] + [x.grad for x in xs]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name", list(CASES))
+def test_routes_agree(dev, name, dtype, monkeypatch):
+    fn, shapes = CASES[name]
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t) or t, lambda t: t):
+        native = _grads(fn, shapes, dtype, dev)
+    assert seen  # saved-tensor hooks see what the node keeps
+    monkeypatch.setattr(_lib, "eager_native", lambda *a: False)
+    for a, b in zip(native, _grads(fn, shapes, dtype, dev)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_changed_input_is_noticed(dev):
+    """An input changed in place between forward and backward raises, as for the registered op."""
+    x = torch.randn(8, 64, device=dev)
+    s = torch.ones(64, device=dev, requires_grad=True)
+    y = rms_norm(x, s)
+    x.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+
+
+def test_eager_native_only_in_plain_eager_mode():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class FM(TorchFunctionMode):
+        def __torch_function__(self, f, types, args=(), kwargs=None):
+            return f(*args, **(kwargs or {}))
+
+    class DM(TorchDispatchMode):
+        def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+            return f(*args, **(kwargs or {}))
+
+    t, p = torch.zeros(2), torch.nn.Parameter(torch.zeros(2))
+    assert _lib.eager_native(t, p, None)
+    for mode in (FM(), DM()):
+        with mode:
+            assert not _lib.eager_native(t)
+    with torch.autograd.forward_ad.dual_level():
+        assert not _lib.eager_native(t)
+    got = []
+    torch.func.vmap(lambda v: got.append(_lib.eager_native(t)) or v)(t)
+    torch.func.grad(lambda v: got.append(_lib.eager_native(t)) or v.sum())(t)
+    assert got == [False, False]
+
+    class Sub(torch.Tensor):
+        pass
+    assert not _lib.eager_native(t.as_subclass(Sub))

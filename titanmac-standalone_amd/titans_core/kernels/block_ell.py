@@ -112,8 +112,7 @@ class BlockELLPattern:
         """Device copy of the grouped forward's balanced tile order for M rows
         (tmac_bell_group_tile_order), cached per (device, M)."""
         import ctypes
-        device = torch.device(device)
-        key = (str(device), int(M))
+        key = (device, M)
         t = self._tord.get(key)
         if t is None:
             L = _lib.lib()
@@ -129,16 +128,15 @@ class BlockELLPattern:
         return t
 
     def device_index(self, device: torch.device) -> dict:
-        device = torch.device(device)
-        key = str(device)
-        if key not in self._dev:
+        idx = self._dev.get(device)
+        if idx is None:
             mk = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
-            self._dev[key] = {
+            idx = self._dev[device] = {
                 "col_idx": mk(self.col_idx.reshape(-1)), "t_ptr": mk(self.t_ptr),
                 "t_row": mk(self.t_row), "t_vblk": mk(self.t_vblk), "order": mk(self.order),
                 "grp": mk(self.grp),
             }
-        return self._dev[key]
+        return idx
 
     def __repr__(self) -> str:
         return (f"BlockELLPattern(n_brow={self.n_brow}, n_bcol={self.n_bcol}, width={self.width}, "
@@ -282,10 +280,10 @@ def _bell_fwd_gelu(x: torch.Tensor, values: torch.Tensor, col_idx: torch.Tensor,
     return y.reshape(shape), z.reshape(shape)
 
 
-bell_fwd_gelu = torch.library.custom_op("titanmac::bell_fwd_gelu", mutates_args=())(_bell_fwd_gelu)
+_bell_fwd_gelu_op = torch.library.custom_op("titanmac::bell_fwd_gelu", mutates_args=())(_bell_fwd_gelu)
 
 
-@bell_fwd_gelu.register_fake
+@_bell_fwd_gelu_op.register_fake
 def _(x, values, col_idx, t_ptr, t_row, t_vblk, order, bias, grp=None, tord=None):
     shape = (*x.shape[:-1], BLOCK * (t_ptr.shape[0] - 1))
     return x.new_empty(shape), x.new_empty(shape)
@@ -461,6 +459,7 @@ def _fwd_backward(ctx, gy):
 
 
 bell_fwd.register_autograd(_fwd_backward, setup_context=_fwd_setup_context)
+_bell_fwd_native = _lib.native_function(_bell_fwd, _fwd_setup_context, _fwd_backward)
 
 
 def _fwd_gelu_setup_context(ctx, inputs, output):
@@ -481,18 +480,27 @@ def _fwd_gelu_backward(ctx, ga, _gz_unused):
     if ga is None:
         ga = torch.zeros_like(z)
     want_b = ctx.has_bias and ctx.needs_input_grad[7]
-    gz, db = bell_gelu_bwd(ga, z, want_b)
+    direct = _lib.direct_call(ga, x, values, z)
+    gz, db = (_bell_gelu_bwd if direct else bell_gelu_bwd)(ga, z, want_b)
     gx = gv = gb = None
     if ctx.needs_input_grad[0]:
-        gx = bell_dx(gz, values, col_idx, ctx.n_bcol).to(x.dtype)
+        gx = (_bell_dx if direct else bell_dx)(gz, values, col_idx, ctx.n_bcol).to(x.dtype)
     if ctx.needs_input_grad[1]:
-        gv = bell_sddmm(x, gz, col_idx, n_brow, width, values.dtype)
+        gv = (_bell_sddmm if direct else bell_sddmm)(x, gz, col_idx, n_brow, width, values.dtype)
     if want_b:
         gb = db.to(ctx.bias_dtype)
     return gx, gv, None, None, None, None, None, gb, None, None
 
 
-bell_fwd_gelu.register_autograd(_fwd_gelu_backward, setup_context=_fwd_gelu_setup_context)
+_bell_fwd_gelu_op.register_autograd(_fwd_gelu_backward, setup_context=_fwd_gelu_setup_context)
+_bell_fwd_gelu_native = _lib.native_function(_bell_fwd_gelu, _fwd_gelu_setup_context, _fwd_gelu_backward,
+                                             all_outputs=True)
+
+
+def bell_fwd_gelu(x, values, col_idx, t_ptr, t_row, t_vblk, order, bias, grp=None, tord=None):
+    """(gelu(z), z) with z = x · W + bias; z is not differentiable (titanmac::bell_fwd_gelu)."""
+    op = _bell_fwd_gelu_native if _lib.eager_native(x, values, bias) else _bell_fwd_gelu_op
+    return op(x, values, col_idx, t_ptr, t_row, t_vblk, order, bias, grp, tord)
 
 
 def block_ell_mm(x: torch.Tensor, values: torch.Tensor, pattern: BlockELLPattern,
@@ -529,7 +537,10 @@ def block_ell_mm(x: torch.Tensor, values: torch.Tensor, pattern: BlockELLPattern
         y, _ = bell_fwd_gelu(x, values, idx["col_idx"], idx["t_ptr"], idx["t_row"], idx["t_vblk"],
                              idx["order"], bias, idx["grp"], tord)
         return y
-    op = _bell_fwd if _lib.direct_call(x, values, bias) else bell_fwd
+    if _lib.direct_call(x, values, bias):
+        op = _bell_fwd
+    else:
+        op = _bell_fwd_native if _lib.eager_native(x, values, bias) else bell_fwd
     y = op(x, values, idx["col_idx"], idx["t_ptr"], idx["t_row"], idx["t_vblk"], idx["order"], bias,
            fuse, idx["grp"], tord)
     if activation == "gelu" and not fuse:

@@ -101,11 +101,14 @@ def _backward(ctx, grad):
 
 
 dwconv_causal.register_autograd(_backward, setup_context=_setup)
+_dwconv_native = _lib.native_function(_dwconv_causal, _setup, _backward)
 
 
 def causal_dwconv(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """Causal depthwise convolution of x [B, T, C] with weight [C, k] (or nn.Conv1d's [C, 1, k])."""
     if weight.dim() == 3:
         weight = weight.reshape(weight.shape[0], weight.shape[2])
-    op = _dwconv_causal if _lib.direct_call(x, weight) else dwconv_causal
+    if _lib.direct_call(x, weight):
+        return _dwconv_causal(x, weight)
+    op = _dwconv_native if _lib.eager_native(x, weight) else dwconv_causal
     return op(x, weight)

@@ -65,8 +65,10 @@ def _rmsnorm_bwd(grad: torch.Tensor, x: torch.Tensor, scale: torch.Tensor,
     g2 = _rows(grad.to(x.dtype))
     M, D = (int(v) for v in x2.shape)
     dx = torch.empty((M, D), dtype=x.dtype, device=dev)
-    dscale = torch.zeros((D,), dtype=torch.float32, device=dev)
-    if M > 0:
+    dscale = torch.empty((D,), dtype=torch.float32, device=dev)
+    if M == 0:
+        dscale.zero_()
+    else:
         L = _lib.lib()
         ws_bytes = ctypes.c_size_t(0)
         _lib.check(L.tmac_rmsnorm_bwd_workspace(M, D, ctypes.byref(ws_bytes)),
@@ -102,9 +104,13 @@ def _backward(ctx, grad_y, grad_rstd):
 
 
 rmsnorm_fwd.register_autograd(_backward, setup_context=_setup)
+_rmsnorm_native = _lib.native_function(_rmsnorm_fwd, _setup, lambda ctx, g: _backward(ctx, g, None))
 
 
 def rms_norm(x: torch.Tensor, scale: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
     """x / sqrt(mean(x², -1) + eps) * scale over the last dimension."""
-    op = _rmsnorm_fwd if _lib.direct_call(x, scale) else rmsnorm_fwd
-    return op(x, scale, float(eps))[0]
+    if _lib.direct_call(x, scale):
+        return _rmsnorm_fwd(x, scale, float(eps))[0]
+    if _lib.eager_native(x, scale):
+        return _rmsnorm_native(x, scale, float(eps))
+    return rmsnorm_fwd(x, scale, float(eps))[0]

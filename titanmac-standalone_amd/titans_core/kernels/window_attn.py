@@ -279,6 +279,7 @@ def _backward(ctx, grad_out, grad_lse):
 
 
 window_attn_fwd.register_autograd(_backward, setup_context=_setup)
+_window_attn_native = _lib.native_function(_window_attn_fwd, _setup, lambda ctx, g: _backward(ctx, g, None))
 
 
 # ---------------------------------------------------------------------------
@@ -566,6 +567,8 @@ def _backward_ex(ctx, grad_out, grad_lse, grad_ws):
 
 
 window_attn_fwd_ex.register_autograd(_backward_ex, setup_context=_setup_ex)
+_window_attn_ex_native = _lib.native_function(_window_attn_fwd_ex, _setup_ex,
+                                              lambda ctx, g: _backward_ex(ctx, g, None, None))
 
 
 def new_dropout_seed() -> int:
@@ -627,13 +630,23 @@ def windowed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window
     need_lse = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad
                                             or v.requires_grad or mask_rg)
     if attn_mask is None and dropout_p == 0.0:
-        op = _window_attn_fwd if _lib.direct_call(q, k, v) else window_attn_fwd
-        out, _ = op(q, k, v, int(window_size), int(n_persistent), bool(causal), code,
-                    int(block_size), float(scale), need_lse)
+        args = (q, k, v, int(window_size), int(n_persistent), bool(causal), code, int(block_size),
+                float(scale), need_lse)
+        if _lib.direct_call(q, k, v):
+            out = _window_attn_fwd(*args)[0]
+        elif need_lse and _lib.eager_native(q, k, v):
+            out = _window_attn_native(*args)
+        else:
+            out = window_attn_fwd(*args)[0]
         return out.transpose(1, 2)
     if seed is None:
         seed = new_dropout_seed() if dropout_p > 0.0 else 0
-    op = _window_attn_fwd_ex if _lib.direct_call(q, k, v, attn_mask) else window_attn_fwd_ex
-    out, _, _ = op(q, k, v, attn_mask, int(window_size), int(n_persistent), bool(causal), code,
-                   int(block_size), float(scale), float(dropout_p), int(seed), need_lse)
+    args = (q, k, v, attn_mask, int(window_size), int(n_persistent), bool(causal), code, int(block_size),
+            float(scale), float(dropout_p), int(seed), need_lse)
+    if _lib.direct_call(q, k, v, attn_mask):
+        out = _window_attn_fwd_ex(*args)[0]
+    elif need_lse and _lib.eager_native(q, k, v, attn_mask):
+        out = _window_attn_ex_native(*args)
+    else:
+        out = window_attn_fwd_ex(*args)[0]
     return out.transpose(1, 2)
