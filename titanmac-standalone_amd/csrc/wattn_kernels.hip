@@ -895,6 +895,11 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void wattn_bwd_kv_kernel(
 // one barrier per tile. Stage = Q and dO tiles (64 rows of 128 bytes, chunks
 // swizzled by swz64: conflict-free for the S/dP operands' 16-byte row reads and
 // the dK/dV operands' transpose reads), then LSE·log2e and −Δ of the 64 queries.
+// The keys that persistent tokens put in the first block (32 of its slices' 128) meet every query
+// tile, so its list ends in a long tail that only one or two of the four waves had work for; at 20
+// heads of 4112 that walk set the kernel's time. The waves share such a tail: each takes every
+// fourth (second) tile by itself and the sums are added through LDS in wave order. dK/dV at 20 heads
+// 108 -> 59 us, at 80 heads 176-184 -> 161-171 us (S = 4112, 16 persistent tokens, bf16).
 // Wave w copies Q and dO rows 16w..16w+15 (two 8-row instructions each); wave 2
 // also copies the 64 LSE values and wave 3 the 64 Δ values, each converting
 // its values in place once they have landed. Rows past S read row S-1 (always
@@ -902,6 +907,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void wattn_bwd_kv_kernel(
 constexpr int kKvStages = 4;
 constexpr int kKvTileB = 64 * 128;             // one 64x64 16-bit tile, bytes
 constexpr int kKvStageB = 2 * kKvTileB + 512;  // Q, dO, LSE·log2e, Δ
+constexpr int kKvTail = 8;  // entries from which a tail of one or two slices is shared by the waves
 
 template <int DT, int FEAT = 0>
 __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
@@ -915,6 +921,9 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     const int32_t* __restrict__ order, WorkMap wm, AttnX ax) {
   constexpr int D = 64;
   constexpr bool CM = (FEAT & kFeatMask) != 0, DR = (FEAT & kFeatDrop) != 0;
+  // With a caller's mask the second copy of the tile's code costs scalar registers and 5 % of the
+  // kernel (45 -> 48 us on packed documents, 80 heads of 2000), and such lists rarely have the tail.
+  constexpr bool kShare = !CM;
   using T = Tile<D>;
   __shared__ __attribute__((aligned(16))) uint16_t ring[kKvStages * kKvStageB / 2];
 
@@ -927,11 +936,12 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;  // uniform
   const int l32 = lane & 31, h = lane >> 5;
   const int grp = (lane >> 4) & 1;
-  const int key = kb * 128 + wave * 32 + l32;  // this lane's key
-  const Span span = mask_col_span(mp, key);     // the queries that see it (partial tiles only)
+  int slice = wave;                     // this wave's 32 keys of the block
+  int key = kb * 128 + slice * 32 + l32;  // this lane's key
+  Span span = mask_col_span(mp, key);     // the queries that see it (partial tiles only)
 
   u32x4 kf[T::kKk], vf[T::kKk];
-  {
+  auto load_kv = [&]() __attribute__((always_inline)) {
     const int kc = min(key, S - 1);
     const uint16_t* kp = K + b * ksb + hd * ksh + static_cast<int64_t>(kc) * kss + 8 * h;
     const uint16_t* vp = V + b * vsb + hd * vsh + static_cast<int64_t>(kc) * vss + 8 * h;
@@ -945,7 +955,8 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
       settle(kf[kk]);
       settle(vf[kk]);
     }
-  }
+  };
+  load_kv();
   const uint16_t* Qbh = Q + b * qsb + hd * qsh;
   const uint16_t* Gbh = dO + b * gsb + hd * gsh;
   const float* lse_bh = lse + static_cast<int64_t>(bh) * S;
@@ -961,6 +972,25 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     e1 = col_ptr[kb + 1];
   }
   const int n = e1 - e0;
+  // The list's tail in which only the first n_sl (1 or 2) key slices are listed, if it is long.
+  int n_main = n, n_sl = 4;
+  if (kShare && n >= 16) {
+    int last1 = -1, last2 = -1;  // last entry listing a slice past the first, past the first two
+    for (int base = 0; base < n; base += 64) {
+      const int ent = base + lane < n ? entries[e0 + base + lane] : 0;
+      const uint64_t b1 = __builtin_amdgcn_ballot_w64((ent & 0x00fc0000) != 0);
+      const uint64_t b2 = __builtin_amdgcn_ballot_w64((ent & 0x00f00000) != 0);
+      if (b1) last1 = base + 63 - __builtin_clzll(b1);
+      if (b2) last2 = base + 63 - __builtin_clzll(b2);
+    }
+    if (n - 1 - last1 >= kKvTail) {
+      n_main = last1 + 1;
+      n_sl = 1;
+    } else if (n - 1 - last2 >= kKvTail) {
+      n_main = last2 + 1;
+      n_sl = 2;
+    }
+  }
   // caller's mask: allowed-query bits of this key in the current and the next tile
   uint64_t wb = 0, wb_next = 0;
   if constexpr (CM) {
@@ -1007,41 +1037,18 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     dvt[dt] = f32x16{};
   }
 
-  for (int i = 0; i < kKvStages - 1 && i < n; ++i) issue(i);
-  for (int i = 0; i < n; ++i) {
-    // this wave's copies of tile i have landed when at most those of the (up
-    // to kKvStages - 2) later tiles already issued are outstanding: four copies
-    // per tile for waves 0-1, five for waves 2-3
-    const int later = min(kKvStages - 2, n - 1 - i);
-    if (wave >= 2) {
-      if (later == 2) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-      else if (later == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else {
-      if (later == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      else if (later == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // This wave's slice into the outputs.
+  auto store_kv = [&]() __attribute__((always_inline)) {
+    if (key < S) {
+      store_row<DT, T::kDt>(dK + b * dksb + hd * dksh + static_cast<int64_t>(key) * dkss, dkt, scale, h);
+      store_row<DT, T::kDt>(dV + b * dvsb + hd * dvsh + static_cast<int64_t>(key) * dvss, dvt, 1.f, h);
     }
-    const uint16_t* st = ring + (i % kKvStages) * (kKvStageB / 2);
-    float* lse2 = reinterpret_cast<float*>(const_cast<uint16_t*>(st) + 2 * (kKvTileB / 2));
-    if (wave >= 2) {
-      // LSE -> LSE·log2e (wave 2) and Δ -> −Δ (wave 3), in place (this wave's
-      // copy has landed)
-      float* v = lse2 + 64 * (wave - 2) + lane;
-      *v = wave == 2 ? lse_log2<CM>(*v) : -*v;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-    // every wave's copies of tile i are in LDS (and converted), and every wave
-    // is done reading the stage the next copies overwrite (tile i-1's)
-    asm volatile("s_barrier" ::: "memory");
-    if (i + kKvStages - 1 < n) issue(i + kKvStages - 1);
+  };
 
-    const int ent = entries[e0 + i];
+  // One listed tile, staged at st, against this wave's slice.
+  auto process = [&](int ent, const uint16_t* st, const float* lse2) __attribute__((always_inline)) {
     const int qt = ent & 0xffff;
-    const int kind = (ent >> (16 + 2 * wave)) & 3;
-    if constexpr (CM) {
-      if (i + 1 < n) wb_next = mask_word(ax, mrow, key, entries[e0 + i + 1] & 0xffff, S);
-    }
+    const int kind = (ent >> (16 + 2 * slice)) & 3;
     if (kind != 0) {
       const uint16_t* q_lds = st;
       const uint16_t* g_lds = st + kKvTileB / 2;
@@ -1096,12 +1103,111 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
                                   });
       }
     }
+  };
+
+  for (int i = 0; i < kKvStages - 1 && i < n_main; ++i) issue(i);
+  for (int i = 0; i < n_main; ++i) {
+    // this wave's copies of tile i have landed when at most those of the (up
+    // to kKvStages - 2) later tiles already issued are outstanding: four copies
+    // per tile for waves 0-1, five for waves 2-3
+    const int later = min(kKvStages - 2, n_main - 1 - i);
+    if (wave >= 2) {
+      if (later == 2) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+      else if (later == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+      if (later == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      else if (later == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const uint16_t* st = ring + (i % kKvStages) * (kKvStageB / 2);
+    float* lse2 = reinterpret_cast<float*>(const_cast<uint16_t*>(st) + 2 * (kKvTileB / 2));
+    if (wave >= 2) {
+      // LSE -> LSE·log2e (wave 2) and Δ -> −Δ (wave 3), in place (this wave's
+      // copy has landed)
+      float* v = lse2 + 64 * (wave - 2) + lane;
+      *v = wave == 2 ? lse_log2<CM>(*v) : -*v;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    // every wave's copies of tile i are in LDS (and converted), and every wave
+    // is done reading the stage the next copies overwrite (tile i-1's)
+    asm volatile("s_barrier" ::: "memory");
+    if (i + kKvStages - 1 < n_main) issue(i + kKvStages - 1);
+    const int ent = entries[e0 + i];
+    if constexpr (CM) {
+      if (i + 1 < n_main) wb_next = mask_word(ax, mrow, key, entries[e0 + i + 1] & 0xffff, S);
+    }
+    process(ent, st, lse2);
     if constexpr (CM) wb = wb_next;
   }
-
-  if (key >= S) return;
-  store_row<DT, T::kDt>(dK + b * dksb + hd * dksh + static_cast<int64_t>(key) * dkss, dkt, scale, h);
-  store_row<DT, T::kDt>(dV + b * dvsb + hd * dvsh + static_cast<int64_t>(key) * dvss, dvt, 1.f, h);
+  if (kShare && n_main < n) {
+    // The tail: waves past the first n_sl write their finished slices, and wave w goes on with slice
+    // w % n_sl, taking every (4 / n_sl)-th entry, copied whole into stage w, which is now its own.
+    if (wave >= n_sl) {
+      store_kv();
+#pragma unroll
+      for (int dt = 0; dt < T::kDt; ++dt) {
+        dkt[dt] = f32x16{};
+        dvt[dt] = f32x16{};
+      }
+      slice = wave & (n_sl - 1);
+      key = kb * 128 + slice * 32 + l32;
+      span = mask_col_span(mp, key);
+      load_kv();
+    }
+    asm volatile("s_barrier" ::: "memory");  // every wave is done with the ring
+    const uint16_t* st = ring + wave * (kKvStageB / 2);
+    float* lse2 = reinterpret_cast<float*>(const_cast<uint16_t*>(st) + 2 * (kKvTileB / 2));
+    const uint32_t sb = ring0 + static_cast<uint32_t>(wave * kKvStageB);
+    for (int i = n_main + wave / n_sl; i < n; i += 4 / n_sl) {
+      const int ent = entries[e0 + i], qt = ent & 0xffff;
+      const uint16_t* qb = Qbh + static_cast<int64_t>(qt) * 64 * qss;
+      const uint16_t* gb = Gbh + static_cast<int64_t>(qt) * 64 * gss;
+      const int lim = S - 1 - qt * 64;
+      int el = lane;  // (opaque: the offsets are formed per tile, not held in registers)
+      asm volatile("" : "+v"(el));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int row = 8 * j + (el >> 3), a = (row >> 1) & 7;
+        const uint32_t r = static_cast<uint32_t>(min(row, lim));
+        const uint32_t ch = 16u * static_cast<uint32_t>((el & 7) ^ (((a & 1) << 2) | (a >> 1)));
+        dma_lds16(qb, r * static_cast<uint32_t>(2 * qss) + ch, sb + j * 1024);
+        dma_lds16(gb, r * static_cast<uint32_t>(2 * gss) + ch, sb + kKvTileB + j * 1024);
+      }
+      const uint32_t qo = 4u * static_cast<uint32_t>(min(qt * 64 + el, S - 1));
+      dma_lds4(lse_bh, qo, sb + 2 * kKvTileB);
+      dma_lds4(dl_bh, qo, sb + 2 * kKvTileB + 256);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lse2[lane] = lse_log2<CM>(lse2[lane]);
+      lse2[64 + lane] = -lse2[64 + lane];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      process(ent, st, lse2);
+    }
+    // The helpers' sums through LDS (lane-major), added in wave order.
+    float* red = reinterpret_cast<float*>(ring);  // 3 x 64 x 64 floats
+    asm volatile("s_barrier" ::: "memory");        // every wave is done with its stage
+    if (wave >= n_sl) {
+#pragma unroll
+      for (int dt = 0; dt < T::kDt; ++dt)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          red[((wave - n_sl) * 64 + dt * 16 + j) * 64 + lane] = dkt[dt][j];
+          red[((wave - n_sl) * 64 + 32 + dt * 16 + j) * 64 + lane] = dvt[dt][j];
+        }
+    }
+    __syncthreads();
+    if (wave >= n_sl) return;
+    for (int w = wave; w + n_sl < 4; w += n_sl) {
+#pragma unroll
+      for (int dt = 0; dt < T::kDt; ++dt)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          dkt[dt][j] += red[(w * 64 + dt * 16 + j) * 64 + lane];
+          dvt[dt][j] += red[(w * 64 + 32 + dt * 16 + j) * 64 + lane];
+        }
+    }
+  }
+  store_kv();
 }
 
 // dQ. Workgroup = (b, h, 128 queries) as in the forward; wave w owns queries
