@@ -89,3 +89,35 @@ def test_eager_native_only_in_plain_eager_mode():
     class Sub(torch.Tensor):
         pass
     assert not _lib.eager_native(t.as_subclass(Sub))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,dh", [(2, 64), (3, 32), (1, 128), (2, 80)])
+@pytest.mark.parametrize("kw", [{}, {"pattern": "blockwin", "causal": False}, {"dropout_p": 0.2}, {"mask": "bool"},
+                                {"mask": "float"}])
+def test_fused_qkv_gradient(dev, dtype, H, dh, kw):
+    """The fused projection's gradient written in place equals the one autograd joins from q, k and v."""
+    from titans_core.kernels.window_attn import _split_heads, windowed_attention_qkv
+    kw = dict(kw)
+    g = torch.Generator().manual_seed(H * dh)
+    B, S = 2, 150
+    qkv = torch.randn(B, S, 3 * H * dh, generator=g).to(dev, dtype)
+    go = torch.randn(B, S, H * dh, generator=g).to(dev, dtype)
+    mask = kw.pop("mask", None)
+    if mask is not None:
+        mask = torch.rand(S, S, generator=g).to(dev)
+        mask = (mask > 0.4) | torch.eye(S, dtype=torch.bool, device=dev) if kw == {} and H == 2 else mask
+    a, b = (qkv.clone().requires_grad_() for _ in range(2))
+    torch.manual_seed(7)
+    ya = windowed_attention_qkv(a, H, 40, 4, attn_mask=mask, **kw)
+    ya.backward(go)
+    torch.manual_seed(7)
+    yb = windowed_attention(*_split_heads(b, H), 40, 4, attn_mask=mask, **kw).transpose(1, 2).reshape(B, S, -1)
+    yb.backward(go)
+    assert torch.equal(ya, yb) and torch.equal(a.grad, b.grad)
+    # an additive mask that needs its own gradient takes the general route
+    if mask is not None and mask.is_floating_point():
+        m = mask.clone().requires_grad_()
+        windowed_attention_qkv(a, H, 40, 4, attn_mask=m).backward(go)
+        assert m.grad is not None

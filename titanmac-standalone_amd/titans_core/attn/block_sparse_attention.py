@@ -34,7 +34,7 @@ import torch.nn as nn
 
 from ..kernels.conv import causal_dwconv
 from ..kernels.linear import Projection
-from ..kernels.window_attn import windowed_attention
+from ..kernels.window_attn import windowed_attention_qkv
 
 
 class BlockSparseAttention(nn.Module):
@@ -86,14 +86,9 @@ class BlockSparseAttention(nn.Module):
         qkv = self.qkv_proj(x)
         if self.use_conv:
             qkv = causal_dwconv(qkv, self._fused_conv_weight(qkv.dtype))
-        q, k, v = qkv.chunk(3, dim=-1)
-        q = q.view(B, T, self.n_heads, self.d_head).transpose(1, 2)
-        k = k.view(B, T, self.n_heads, self.d_head).transpose(1, 2)
-        v = v.view(B, T, self.n_heads, self.d_head).transpose(1, 2)
-        out = windowed_attention(q, k, v, self.window_size, self.n_persistent, self.causal,
-                                 pattern="blockwin", block_size=self.block_size, scale=self.scale,
-                                 dropout_p=self.dropout_p if self.training else 0.0)
-        out = out.transpose(1, 2).reshape(B, T, self.d_model)
+        out = windowed_attention_qkv(qkv, self.n_heads, self.window_size, self.n_persistent, self.causal,
+                                     pattern="blockwin", block_size=self.block_size, scale=self.scale,
+                                     dropout_p=self.dropout_p if self.training else 0.0)
         return self.dropout(self.out_proj(out))
 
 

@@ -22,7 +22,7 @@ import torch
 import torch.nn as nn
 
 from ..kernels.linear import Projection
-from ..kernels.window_attn import windowed_attention
+from ..kernels.window_attn import windowed_attention_qkv
 
 
 @dataclass
@@ -124,13 +124,8 @@ class WindowedAttention(nn.Module):
         """
         B, T, D = x.shape
         qkv = self.qkv_proj(x)
-        q, k, v = qkv.chunk(3, dim=-1)
-        # [B, T, d] -> [B, H, T, dh] views (no copy): strides (T*3d, dh, 3d, 1)
-        q = q.view(B, T, self.n_heads, self.d_head).transpose(1, 2)
-        k = k.view(B, T, self.n_heads, self.d_head).transpose(1, 2)
-        v = v.view(B, T, self.n_heads, self.d_head).transpose(1, 2)
+        # the kernels read q, k and v through their strides: no copy
         p = self.dropout_p if self.training else 0.0
-        out = windowed_attention(q, k, v, self.window_size, self.num_persistent, self.causal,
-                                 attn_mask=attn_mask, dropout_p=p)
-        out = out.transpose(1, 2).reshape(B, T, self.d_model)
+        out = windowed_attention_qkv(qkv, self.n_heads, self.window_size, self.num_persistent, self.causal,
+                                     attn_mask=attn_mask, dropout_p=p)
         return self.dropout(self.out_proj(out))

@@ -213,6 +213,13 @@ def _window_attn_bwd(grad_out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v
                      scale: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """(dq, dk, dv), each [B, H, S, dh] (transposed views of [B, S, H, dh] buffers), from
     grad_out and out [B, S, H, dh] and lse [B, H, S] of window_attn_fwd."""
+    return _attn_bwd_into(None, grad_out, q, k, v, out, lse, window_size, n_persistent, causal, pattern,
+                          block_size, scale)
+
+
+def _attn_bwd_into(grads, grad_out, q, k, v, out, lse, window_size, n_persistent, causal, pattern,
+                   block_size, scale):
+    """_window_attn_bwd, into the [B, S, H, dh] views `grads` of dq, dk, dv (None: new buffers)."""
     _check_qkv(q, k, v)
     B, H, S, dh = (int(s) for s in q.shape)
     if out.shape != (B, S, H, dh) or grad_out.shape != (B, S, H, dh):
@@ -225,7 +232,8 @@ def _window_attn_bwd(grad_out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v
             or grad_out.data_ptr() % 16:
         grad_out = grad_out.contiguous()
     lse = lse.contiguous()
-    grads = [torch.empty((B, S, H, dh), dtype=q.dtype, device=dev) for _ in range(3)]
+    if grads is None:
+        grads = [torch.empty((B, S, H, dh), dtype=q.dtype, device=dev) for _ in range(3)]
     views = [g.permute(0, 2, 1, 3) for g in grads]
     if B * H * S == 0:
         return tuple(views)
@@ -465,6 +473,13 @@ def _window_attn_bwd_ex(grad_out: torch.Tensor, q: torch.Tensor, k: torch.Tensor
     own shape and dtype, as SDPA's autograd gives it: dS = P * (dP - Delta) of every
     (b, h, q, k), summed over the mask's broadcast dimensions in a fixed order
     (tmac_wattn_mask_grad_reduce); else an empty tensor."""
+    return _attn_bwd_ex_into(None, grad_out, q, k, v, out, lse, mask, ws, window_size, n_persistent, causal,
+                             pattern, block_size, scale, dropout_p, seed, mask_grad)
+
+
+def _attn_bwd_ex_into(grads, grad_out, q, k, v, out, lse, mask, ws, window_size, n_persistent, causal,
+                      pattern, block_size, scale, dropout_p, seed, mask_grad=False):
+    """_window_attn_bwd_ex, into the [B, S, H, dh] views `grads` of dq, dk, dv (None: new buffers)."""
     _check_qkv(q, k, v)
     B, H, S, dh = (int(s) for s in q.shape)
     if out.shape != (B, S, H, dh) or grad_out.shape != (B, S, H, dh):
@@ -477,7 +492,8 @@ def _window_attn_bwd_ex(grad_out: torch.Tensor, q: torch.Tensor, k: torch.Tensor
             or grad_out.data_ptr() % 16:
         grad_out = grad_out.contiguous()
     lse = lse.contiguous()
-    grads = [torch.empty((B, S, H, dh), dtype=q.dtype, device=dev) for _ in range(3)]
+    if grads is None:
+        grads = [torch.empty((B, S, H, dh), dtype=q.dtype, device=dev) for _ in range(3)]
     views = [g.permute(0, 2, 1, 3) for g in grads]
     if mask_grad and (mask is None or mask.dtype == torch.bool):
         raise ValueError("a mask gradient exists for an additive float attn_mask only")
@@ -577,6 +593,13 @@ def new_dropout_seed() -> int:
     return int(torch.randint(0, 2**63 - 1, (), dtype=torch.int64).item())
 
 
+def _check_pattern(S: int, window_size: int, n_persistent: int, code: int) -> None:
+    if n_persistent > S or (code == _lib.PATTERN_BAND and n_persistent == S):
+        raise ValueError(f"num_persistent_tokens ({n_persistent}) must be < seq_len ({S})")
+    if window_size < 0:
+        raise ValueError(f"window_size must be non-negative, got {window_size}")
+
+
 def windowed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window_size: int,
                        n_persistent: int, causal: bool = True, pattern="band",
                        block_size: int = 64, scale: Optional[float] = None,
@@ -620,10 +643,7 @@ def windowed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window
     S = q.shape[2]
     code = _pattern_code(pattern)
     if attn_mask is None:
-        if n_persistent > S or (code == _lib.PATTERN_BAND and n_persistent == S):
-            raise ValueError(f"num_persistent_tokens ({n_persistent}) must be < seq_len ({S})")
-        if window_size < 0:
-            raise ValueError(f"window_size must be non-negative, got {window_size}")
+        _check_pattern(S, window_size, n_persistent, code)
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
     mask_rg = attn_mask is not None and attn_mask.requires_grad
@@ -650,3 +670,75 @@ def windowed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window
     else:
         out = window_attn_fwd_ex(*args)[0]
     return out.transpose(1, 2)
+
+
+# ---------------------------------------------------------------------------
+# Attention on a fused qkv projection (the modules' training step).
+
+def _split_heads(qkv: torch.Tensor, H: int):
+    """q, k, v as [B, H, S, dh] views of a projection output [B, S, 3 H dh] (no copy)."""
+    B, S, D3 = qkv.shape
+    return [t.view(B, S, H, D3 // (3 * H)).transpose(1, 2) for t in qkv.chunk(3, dim=-1)]
+
+
+class _FusedQKV(torch.autograd.Function):
+    """windowed_attention of the three parts of qkv as one node: its backward writes dq, dk and dv
+    straight into the fused projection's gradient, where autograd's chain of views would concatenate
+    three buffers (36 us of a 32 x 560 x 640 bf16 step, and a dozen nodes of host time)."""
+
+    @staticmethod
+    def forward(ctx, qkv, mask, H, args, dropout_p, seed):
+        q, k, v = _split_heads(qkv, H)
+        ws = None
+        if mask is None and dropout_p == 0.0:
+            out, lse = _window_attn_fwd(q, k, v, *args, True)
+        else:
+            out, lse, ws = _window_attn_fwd_ex(q, k, v, mask, *args, dropout_p, seed, True)
+        ctx.save_for_backward(qkv, out, lse, mask, ws)
+        ctx.call = (H, args, dropout_p, seed)
+        return out.flatten(2)
+
+    @staticmethod
+    def backward(ctx, grad):
+        qkv, out, lse, mask, ws = ctx.saved_tensors
+        H, args, dropout_p, seed = ctx.call
+        q, k, v = _split_heads(qkv, H)
+        g = grad.reshape(out.shape)
+        if not _lib.direct_call(grad, qkv):  # a backward that is itself recorded: the registered ops
+            if ws is None:
+                ds = window_attn_bwd(g, q, k, v, out, lse, *args)
+            else:
+                ds = window_attn_bwd_ex(g, q, k, v, out, lse, mask, ws, *args, dropout_p, seed)[:3]
+            return torch.cat([d.transpose(1, 2).flatten(2) for d in ds], dim=-1), None, None, None, None, None
+        B, S, _, dh = out.shape
+        dqkv = torch.empty((B, S, 3, H, dh), dtype=qkv.dtype, device=qkv.device)
+        grads = dqkv.unbind(2)
+        if ws is None:
+            _attn_bwd_into(grads, g, q, k, v, out, lse, *args)
+        else:
+            _attn_bwd_ex_into(grads, g, q, k, v, out, lse, mask, ws, *args, dropout_p, seed)
+        return dqkv.view(B, S, 3 * H * dh), None, None, None, None, None
+
+
+def windowed_attention_qkv(qkv: torch.Tensor, n_heads: int, window_size: int, n_persistent: int,
+                           causal: bool = True, pattern="band", block_size: int = 64,
+                           scale: Optional[float] = None, attn_mask: Optional[torch.Tensor] = None,
+                           dropout_p: float = 0.0) -> torch.Tensor:
+    """windowed_attention of the q, k and v parts of a fused projection's output [B, S, 3 d], heads merged
+    again: [B, S, d]."""
+    B, S, D3 = qkv.shape
+    dh = D3 // (3 * n_heads)
+    code = _pattern_code(pattern)
+    if (torch.is_grad_enabled() and qkv.requires_grad and dh in HEAD_DIMS and qkv.is_cuda
+            and (attn_mask is None or not attn_mask.requires_grad) and B * S > 0
+            and _lib.eager_native(qkv, attn_mask)):
+        if attn_mask is None:
+            _check_pattern(S, window_size, n_persistent, code)
+        args = (int(window_size), int(n_persistent), bool(causal), code, int(block_size),
+                float(1.0 / math.sqrt(dh) if scale is None else scale))
+        seed = new_dropout_seed() if dropout_p > 0.0 else 0
+        return _FusedQKV.apply(qkv, attn_mask, n_heads, args, float(dropout_p), seed)
+    q, k, v = _split_heads(qkv, n_heads)
+    out = windowed_attention(q, k, v, window_size, n_persistent, causal, pattern, block_size, scale,
+                             attn_mask, dropout_p)
+    return out.transpose(1, 2).reshape(B, S, D3 // 3)
