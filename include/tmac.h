@@ -639,6 +639,16 @@ int tmac_silu_bwd(const void* d_dh, const void* d_z, void* d_dz, int64_t n, int 
 int tmac_mse_grad(const void* d_y, const void* d_v, void* d_dy, int64_t n, float coef, int dtype,
                   void* stream);
 
+/* Backward of an MLP's hidden layer, 16-bit: with a = gelu(z) the input of a Block-ELL layer W2
+ * [K, N], gZ[M, K] = (dY · W2ᵀ, rounded to dtype) ⊙ GELU'(Z), the product of tmac_bell_dx and
+ * tmac_bell_gelu_bwd in one pass, and (d_dbias non-NULL) dbias[K] = the fp32 column sums of gZ
+ * before its rounding, in a fixed order. d_ws: tmac_bell_dx_gelu_workspace bytes when d_dbias is given. */
+int tmac_bell_dx_gelu_workspace(int M, int n_brow, size_t* ws_bytes);
+int tmac_bell_dx_gelu(const void* d_dY, int64_t lddy, const void* d_vals, const int32_t* d_col_idx,
+                      const void* d_Z, int64_t ldz, void* d_gZ, int64_t ldgz, float* d_dbias,
+                      void* d_ws, size_t ws_bytes, int M, int n_brow, int n_bcol, int width, int dtype,
+                      void* stream);
+
 /* ------------------------------------------------------------------------
  * Dense projections: nn.Linear without bias on 16-bit inputs (fp32
  * accumulation), the qkv and output projections of the attention modules

@@ -81,13 +81,20 @@ __device__ __forceinline__ void dma16(const uint16_t* src, uint16_t* lds_base) {
   __builtin_amdgcn_global_load_lds(src, (lds_void*)(lds_base), 16, 0, 0);
 }
 
-template <int DT, bool FWD>
+// GB (dX of an MLP's second layer): the epilogue multiplies the input gradient, rounded as the plain
+// kernel stores it, by GELU'(Z) of the first layer's saved pre-activation and stores that product
+// (the gradient of Z), and with `part` the tile's fp32 column sums of it (the first layer's bias gradient,
+// one row of partial sums per 256 rows, added by column_sum_kernel). The separate pass over the
+// gradient (bell_gelu_bwd_kernel) read and wrote 335 MB more at 32768 x 2560: 103 + 89 us for the two
+// kernels, 161 us here.
+template <int DT, bool FWD, bool GB = false>
 __global__ __launch_bounds__(256, 2) void bell_gemm_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ vals,
     const int32_t* __restrict__ t_ptr, const int32_t* __restrict__ in_blk,
     const int32_t* __restrict__ t_vblk, const int32_t* __restrict__ order,
     const uint16_t* __restrict__ bias, int epi, uint16_t* __restrict__ Y, int64_t ldy,
-    uint16_t* __restrict__ Z, int64_t ldz, int M, int n_out, int width, int n_mtiles, int per_xcd) {
+    uint16_t* __restrict__ Z, int64_t ldz, int M, int n_out, int width, int n_mtiles, int per_xcd,
+    float* __restrict__ part = nullptr) {
   // Two buffers, each the activation tile (kBM x 64, xswz) and the weight
   // block (64 x 64, swz64); the epilogue's four per-wave 64x64 staging tiles
   // (pitch kPitch) reuse the same memory.
@@ -163,6 +170,16 @@ __global__ __launch_bounds__(256, 2) void bell_gemm_kernel(
     bin = __builtin_amdgcn_readlane(win_in, i - win_base);
     bw = __builtin_amdgcn_readlane(win_w, i - win_base);
   };
+
+  // GB: this lane's Z, rows 8 it + lane / 8 of the wave's 64 and columns 8 (lane % 8)..+7, in flight
+  // with the first tiles (rows past M read row M-1 and are neither stored nor summed)
+  const int64_t colz = static_cast<int64_t>(ob) * 64 + 8 * dpos;
+  u32x4 zz[GB ? 8 : 1];
+  if constexpr (GB) {
+#pragma unroll
+    for (int it = 0; it < 8; ++it)
+      zz[it] = ldg16(Z + static_cast<int64_t>(min(m_base + 8 * it + drow, M - 1)) * ldz + colz);
+  }
 
   f32x16 acc[2][2];
 #pragma unroll
@@ -245,6 +262,68 @@ __global__ __launch_bounds__(256, 2) void bell_gemm_kernel(
       compute(smem0);
       __syncthreads();
     }
+  }
+
+  if constexpr (GB) {
+    uint16_t* st = smem0 + wave * kTileElems;
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+        for (int jg = 0; jg < 4; ++jg) {
+          u32x2 packed;
+          packed.x = Mfma<DT>::pack2(acc[mi][ni][4 * jg], acc[mi][ni][4 * jg + 1]);
+          packed.y = Mfma<DT>::pack2(acc[mi][ni][4 * jg + 2], acc[mi][ni][4 * jg + 3]);
+          *reinterpret_cast<u32x2*>(st + (32 * mi + l32) * kPitch + 32 * ni + 8 * jg + 4 * h) = packed;
+        }
+    __syncthreads();
+    float sum[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sum[k] = 0.f;
+    auto rows8 = [&](int it, bool valid) __attribute__((always_inline)) {
+      const u32x4 a4 = lds16(st + (8 * it + drow) * kPitch + 8 * dpos);
+      const uint32_t aw[4] = {a4.x, a4.y, a4.z, a4.w};
+      const uint32_t zw[4] = {zz[it].x, zz[it].y, zz[it].z, zz[it].w};
+      uint32_t ow[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float g0 = Mfma<DT>::to_f32(static_cast<uint16_t>(aw[i] & 0xffff)) *
+                         gelu_erf_grad(Mfma<DT>::to_f32(static_cast<uint16_t>(zw[i] & 0xffff)));
+        const float g1 = Mfma<DT>::to_f32(static_cast<uint16_t>(aw[i] >> 16)) *
+                         gelu_erf_grad(Mfma<DT>::to_f32(static_cast<uint16_t>(zw[i] >> 16)));
+        ow[i] = Mfma<DT>::pack2(g0, g1);
+        sum[2 * i] += valid ? g0 : 0.f;
+        sum[2 * i + 1] += valid ? g1 : 0.f;
+      }
+      if (valid)
+        stg16_nt(Y + static_cast<int64_t>(m_base + 8 * it + drow) * ldy + colz, u32x4{ow[0], ow[1], ow[2], ow[3]});
+    };
+    if (m_tile0 + kBM <= M) {
+#pragma unroll
+      for (int it = 0; it < 8; ++it) rows8(it, true);
+    } else {
+#pragma unroll
+      for (int it = 0; it < 8; ++it) rows8(it, m_base + 8 * it + drow < M);
+    }
+    if (!part) return;
+    // the wave's column sums (lanes of one column group), then the four waves' in wave order
+    float* red = reinterpret_cast<float*>(smem1);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      sum[k] += __shfl_xor(sum[k], 8);
+      sum[k] += __shfl_xor(sum[k], 16);
+      sum[k] += __shfl_xor(sum[k], 32);
+    }
+    if (lane < 8) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) red[wave * 64 + 8 * lane + k] = sum[k];
+    }
+    __syncthreads();
+    if (tid < 64)
+      part[static_cast<int64_t>(mtile) * n_out * 64 + static_cast<int64_t>(ob) * 64 + tid] =
+          ((red[tid] + red[64 + tid]) + red[128 + tid]) + red[192 + tid];
+    return;
   }
 
   // Epilogue: bias, activation, conversion, then pack through this wave's LDS
@@ -1445,11 +1524,11 @@ int bell_fwd_impl(const void* d_X, int64_t ldx, const void* d_vals, const int32_
   if (dtype == TMAC_BF16)
     hipLaunchKernelGGL((bell_gemm_kernel<TMAC_BF16, true>), dim3(8 * per_xcd), dim3(256), 0, s, X,
                        ldx, V, d_t_ptr, d_t_row, d_t_vblk, d_order, b, epi, Y, ldy, Z, ldz, M, n_bcol,
-                       width, n_mtiles, per_xcd);
+                       width, n_mtiles, per_xcd, static_cast<float*>(nullptr));
   else
     hipLaunchKernelGGL((bell_gemm_kernel<TMAC_F16, true>), dim3(8 * per_xcd), dim3(256), 0, s, X,
                        ldx, V, d_t_ptr, d_t_row, d_t_vblk, d_order, b, epi, Y, ldy, Z, ldz, M, n_bcol,
-                       width, n_mtiles, per_xcd);
+                       width, n_mtiles, per_xcd, static_cast<float*>(nullptr));
   return launch_status();
 }
 
@@ -1600,11 +1679,60 @@ extern "C" int tmac_bell_dx(const void* d_dY, int64_t lddy, const void* d_vals,
   if (dtype == TMAC_BF16)
     hipLaunchKernelGGL((bell_gemm_kernel<TMAC_BF16, false>), dim3(8 * per_xcd), dim3(256), 0, s,
                        dY, lddy, V, nullptr, d_col_idx, nullptr, nullptr, nullptr, 0, dX, lddx, nullptr,
-                       0, M, n_brow, width, n_mtiles, per_xcd);
+                       0, M, n_brow, width, n_mtiles, per_xcd, static_cast<float*>(nullptr));
   else
     hipLaunchKernelGGL((bell_gemm_kernel<TMAC_F16, false>), dim3(8 * per_xcd), dim3(256), 0, s,
                        dY, lddy, V, nullptr, d_col_idx, nullptr, nullptr, nullptr, 0, dX, lddx, nullptr,
-                       0, M, n_brow, width, n_mtiles, per_xcd);
+                       0, M, n_brow, width, n_mtiles, per_xcd, static_cast<float*>(nullptr));
+  return launch_status();
+}
+
+extern "C" int tmac_bell_dx_gelu_workspace(int M, int n_brow, size_t* ws_bytes) {
+  if (!ws_bytes) return TMAC_ERR_NULL;
+  if (M <= 0 || n_brow <= 0) return TMAC_ERR_SHAPE;
+  *ws_bytes = static_cast<size_t>((M + kBM - 1) / kBM) * n_brow * 64 * sizeof(float);
+  return TMAC_OK;
+}
+
+extern "C" int tmac_bell_dx_gelu(const void* d_dY, int64_t lddy, const void* d_vals,
+                                 const int32_t* d_col_idx, const void* d_Z, int64_t ldz, void* d_gZ,
+                                 int64_t ldgz, float* d_dbias, void* d_ws, size_t ws_bytes, int M,
+                                 int n_brow, int n_bcol, int width, int dtype, void* stream) {
+  if (!d_dY || !d_vals || !d_col_idx || !d_Z || !d_gZ || (d_dbias && !d_ws)) return TMAC_ERR_NULL;
+  int st = check_bell_shape(M, n_brow, n_bcol, width);
+  if (st != TMAC_OK) return st;
+  if (dtype != TMAC_BF16 && dtype != TMAC_F16) return TMAC_ERR_DTYPE;
+  const int64_t K = 64ll * n_brow, N = 64ll * n_bcol;
+  if (lddy < N || ldz < K || ldgz < K) return TMAC_ERR_SHAPE;
+  if (!aligned16(d_dY) || !aligned16(d_vals) || !aligned16(d_Z) || !aligned16(d_gZ) || (lddy % 8) ||
+      (ldz % 8) || (ldgz % 8))
+    return TMAC_ERR_ALIGN;
+  const int n_mtiles = (M + kBM - 1) / kBM;
+  const int64_t total = static_cast<int64_t>(n_mtiles) * n_brow;
+  if (total > (1ll << 30)) return TMAC_ERR_SHAPE;
+  if (d_dbias) {
+    if (ws_bytes < static_cast<size_t>(n_mtiles) * K * sizeof(float)) return TMAC_ERR_WORKSPACE;
+    if (!aligned16(d_ws)) return TMAC_ERR_ALIGN;
+  }
+  const int per_xcd = static_cast<int>((total + 7) / 8);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const auto* dY = static_cast<const uint16_t*>(d_dY);
+  const auto* V = static_cast<const uint16_t*>(d_vals);
+  auto* Z = static_cast<uint16_t*>(const_cast<void*>(d_Z));  // read only
+  auto* gZ = static_cast<uint16_t*>(d_gZ);
+  float* part = d_dbias ? static_cast<float*>(d_ws) : nullptr;
+  if (dtype == TMAC_BF16)
+    hipLaunchKernelGGL((bell_gemm_kernel<TMAC_BF16, false, true>), dim3(8 * per_xcd), dim3(256), 0, s, dY,
+                       lddy, V, nullptr, d_col_idx, nullptr, nullptr, nullptr, 0, gZ, ldgz, Z, ldz, M, n_brow,
+                       width, n_mtiles, per_xcd, part);
+  else
+    hipLaunchKernelGGL((bell_gemm_kernel<TMAC_F16, false, true>), dim3(8 * per_xcd), dim3(256), 0, s, dY,
+                       lddy, V, nullptr, d_col_idx, nullptr, nullptr, nullptr, 0, gZ, ldgz, Z, ldz, M, n_brow,
+                       width, n_mtiles, per_xcd, part);
+  st = launch_status();
+  if (st != TMAC_OK || !d_dbias) return st;
+  hipLaunchKernelGGL(column_sum_kernel, dim3(static_cast<unsigned>((K + 63) / 64)), dim3(256), 0, s, part,
+                     d_dbias, K, n_mtiles, int64_t{0});
   return launch_status();
 }
 

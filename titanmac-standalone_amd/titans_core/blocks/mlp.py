@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from ..kernels.block_ell import BlockELLLinear
+from ..kernels.block_ell import BlockELLLinear, block_ell_mlp
 
 
 class MLPBlock(nn.Module):
@@ -73,7 +73,7 @@ class MLPBlock(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.block_ell:
-            hidden = self.fc1(x, activation="gelu")
+            y = block_ell_mlp(x, self.fc1, self.fc2)
         else:
-            hidden = self.activation(self.fc1(x))
-        return self.dropout(self.fc2(hidden))
+            y = self.fc2(self.activation(self.fc1(x)))
+        return self.dropout(y)

@@ -82,6 +82,8 @@ SIGNATURES = {
                           _vp, _vp, _vp, _i, _i, _vp, _vp],
     "tmac_wattn_mask_lists": [_vp, _i, _vp],
     "tmac_wattn_mask_grad_reduce": [_vp, _i, _i, _i, _i, _i, _vp, _vp],
+    "tmac_bell_dx_gelu_workspace": [_i, _i, ctypes.POINTER(_sz)],
+    "tmac_bell_dx_gelu": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp],
     "tmac_linear_fwd": [_vp, _i64, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
     "tmac_linear_dx": [_vp, _i64, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
     "tmac_linear_wgrad_workspace": [_i, _i, _i, ctypes.POINTER(_sz)],

@@ -548,6 +548,103 @@ def block_ell_mm(x: torch.Tensor, values: torch.Tensor, pattern: BlockELLPattern
     return y
 
 
+def _bell_dx_gelu(gy: torch.Tensor, values: torch.Tensor, col_idx: torch.Tensor, z: torch.Tensor,
+                  with_bias: bool) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """(gz, dbias): gz = (gy · Wᵀ) ⊙ GELU'(z) for [M, ...] 16-bit rows, M > 0, and the fp32 column sums
+    of gz, in one pass (tmac_bell_dx_gelu)."""
+    import ctypes
+    n_brow, width = int(values.shape[0]), int(values.shape[1])
+    K, N = BLOCK * n_brow, gy.shape[-1]
+    dev = _lib.require_device(gy, values, col_idx, z, what="bell_dx_gelu")
+    g2, ldg = _rows(gy.to(values.dtype), N)
+    z2, ldz = _rows(z, K)
+    M = g2.shape[0]
+    gz = torch.empty((M, K), dtype=values.dtype, device=dev)
+    db, ws = None, None
+    L = _lib.lib()
+    if with_bias:
+        nb = ctypes.c_size_t(0)
+        _lib.check(L.tmac_bell_dx_gelu_workspace(M, n_brow, ctypes.byref(nb)), "tmac_bell_dx_gelu_workspace")
+        ws = torch.empty(nb.value // 4, dtype=torch.float32, device=dev)
+        db = torch.empty(K, dtype=torch.float32, device=dev)
+    with _lib.device_guard(dev):
+        rc = L.tmac_bell_dx_gelu(_lib.ptr(g2), ldg, _lib.ptr(values.contiguous()), _lib.ptr(col_idx),
+                                 _lib.ptr(z2), ldz, _lib.ptr(gz), K, _lib.ptr(db), _lib.ptr(ws),
+                                 ws.numel() * 4 if ws is not None else 0, M, n_brow, N // BLOCK, width,
+                                 _lib.dtype_code(values.dtype), _lib.stream_ptr(dev))
+    _lib.check(rc, "tmac_bell_dx_gelu")
+    return gz.reshape(z.shape), db
+
+
+class _MLP(torch.autograd.Function):
+    """fc2(gelu(fc1(x))) of two Block-ELL layers as one node, so that the backward forms the hidden
+    layer's gradient in fc2's dX kernel (tmac_bell_dx_gelu)."""
+
+    @staticmethod
+    def forward(ctx, x, v1, b1, v2, b2, i1, i2):
+        a, z = _bell_fwd_gelu(x, v1, i1["col_idx"], i1["t_ptr"], i1["t_row"], i1["t_vblk"], i1["order"], b1,
+                              i1["grp"], i1["tord"])
+        y = _bell_fwd(a, v2, i2["col_idx"], i2["t_ptr"], i2["t_row"], i2["t_vblk"], i2["order"], b2, False,
+                      i2["grp"], i2["tord"])
+        ctx.save_for_backward(x, v1, z, a, v2, i1["col_idx"], i2["col_idx"])
+        ctx.n_bcol = (i1["t_ptr"].numel() - 1, i2["t_ptr"].numel() - 1)
+        ctx.bias_dtypes = [None if b is None else b.dtype for b in (b1, b2)]
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, v1, z, a, v2, c1, c2 = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        direct = _lib.direct_call(gy, x, v1, v2)  # else the backward is itself recorded: registered ops
+        dx, sddmm = (_bell_dx, _bell_sddmm) if direct else (bell_dx, bell_sddmm)
+        gx = g1 = gb1 = g2 = gb2 = None
+        if need[0] or need[1] or need[2]:
+            if direct:
+                gz, db = _bell_dx_gelu(gy, v2, c2, z, need[2])
+            else:
+                gz, db = bell_gelu_bwd(dx(gy, v2, c2, ctx.n_bcol[1]), z, need[2])
+            if need[0]:
+                gx = dx(gz, v1, c1, ctx.n_bcol[0])
+            if need[1]:
+                g1 = sddmm(x, gz, c1, v1.shape[0], v1.shape[1], v1.dtype)
+            if need[2]:
+                gb1 = db.to(ctx.bias_dtypes[0])
+        if need[3]:
+            g2 = sddmm(a, gy, c2, v2.shape[0], v2.shape[1], v2.dtype)
+        if need[4]:
+            gb2 = _bell_bias_grad(gy.reshape(-1, gy.shape[-1])).to(ctx.bias_dtypes[1])
+        return gx, g1, gb1, g2, gb2, None, None
+
+
+def _plain_layer(m: nn.Module) -> bool:
+    """A BlockELLLinear whose call is only its forward: nothing observes or replaces it."""
+    return (type(m) is BlockELLLinear and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
+
+
+def block_ell_mlp(x: torch.Tensor, fc1: "BlockELLLinear", fc2: "BlockELLLinear") -> torch.Tensor:
+    """fc2(gelu(fc1(x))). A 16-bit training step of two plain layers is one autograd node (_MLP); every
+    other call runs the layers one after the other."""
+    if (x.is_cuda and torch.is_grad_enabled() and _plain_layer(fc1) and _plain_layer(fc2) and x.numel() > 0
+            and not torch.nn.modules.module._has_any_global_hook()):
+        ts = (x, fc1.values, fc1.bias, fc2.values, fc2.bias)
+        if _lib.eager_native(*ts) and any(t is not None and t.requires_grad for t in ts):
+            if torch.is_autocast_enabled("cuda"):
+                dt = torch.get_autocast_dtype("cuda")
+                if dt in (torch.bfloat16, torch.float16):
+                    ts = tuple(None if t is None else t.to(dt) for t in ts)
+            if (ts[0].dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == fc1.in_features
+                    and all(t is None or (t.dtype == ts[0].dtype and t.device == x.device) for t in ts)):
+                M = x.numel() // x.shape[-1]
+                idx = []
+                for p in (fc1.pattern, fc2.pattern):
+                    i = dict(p.device_index(x.device))
+                    i["tord"] = p.tile_order(M, x.device) if M > 64 else None
+                    idx.append(i)
+                return _MLP.apply(*ts, *idx)
+    return fc2(fc1(x, activation="gelu"))
+
+
 # ---------------------------------------------------------------------------
 # Module
 # ---------------------------------------------------------------------------
