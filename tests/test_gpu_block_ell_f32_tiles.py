@@ -1,0 +1,37 @@
+"""fp32 Block-ELL products at the edges of both tile heights (64 rows for small grids, 128 for large)."""
+import pytest
+import torch
+
+from titans_core.kernels import block_ell as kb
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,n_brow,n_bcol,width", [(1, 2, 3, 1), (63, 3, 5, 2), (64, 3, 5, 5), (65, 1, 4, 4), (127, 3, 2, 2),
+                                                   (129, 3, 5, 3), (6529, 3, 40, 10), (6528, 40, 3, 2)])
+def test_f32_products(dev, M, n_brow, n_bcol, width):
+    g = torch.Generator().manual_seed(M)
+    pat = kb.BlockELLPattern.sample(2, n_brow, n_bcol, width)
+    x = torch.randn(M, 64 * n_brow, generator=g).to(dev)
+    gy = torch.randn(M, 64 * n_bcol, generator=g).to(dev)
+    v = torch.randn(n_brow, width, 64, 64, generator=g).to(dev)
+    b = torch.randn(64 * n_bcol, generator=g).to(dev)
+    ci = torch.from_numpy(pat.col_idx).to(dev)
+    W = torch.zeros(n_brow, n_bcol, 64, 64, dtype=torch.float64, device=dev)
+    W[torch.arange(n_brow, device=dev)[:, None], ci.long()] = v.double()
+    W = W.permute(0, 2, 1, 3).reshape(64 * n_brow, 64 * n_bcol)
+
+    def close(got, a, w, add=None):
+        """fp32 sums in any order: (K + 2) 2^-24 times the sum of magnitudes."""
+        ref, mag = a.double() @ w, a.double().abs() @ w.abs()
+        if add is not None:
+            ref, mag = ref + add.double(), mag + add.double().abs()
+        assert torch.all((got.double() - ref).abs() <= (w.shape[0] + 2) * 2.0 ** -24 * mag)
+    close(kb.block_ell_mm(x, v, pat, b), x, W, b)
+    close(kb._bell_dx(gy, v, ci.reshape(-1), n_bcol), gy, W.t())
+    dv = kb._bell_sddmm(x, gy, ci.reshape(-1), n_brow, width, torch.float32)
+    ref = (x.double().t() @ gy.double()).reshape(n_brow, 64, n_bcol, 64).permute(0, 2, 1, 3)
+    mag = (x.double().abs().t() @ gy.double().abs()).reshape(n_brow, 64, n_bcol, 64).permute(0, 2, 1, 3)
+    rows = torch.arange(n_brow, device=dev)[:, None]
+    err = (dv.double() - ref[rows, ci.long()]).abs()
+    assert torch.all(err <= (M + 2) * 2.0 ** -24 * mag[rows, ci.long()])

@@ -1054,31 +1054,32 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
 // fp32 path (fp32 modules without autocast): the same three products on
 // v_mfma_f32_32x32x2_f32, fp32 products and fp32 accumulation.
 //
-// Gather GEMM (forward and dX): a workgroup owns a 128-row by 64-column output
+// Gather GEMM (forward and dX): a workgroup owns a BM-row (128 or 64, f32_rows) by 64-column output
 // tile and walks the same list as the 16-bit kernel. Per list entry it stages
-// the 128x64 activation tile (row-major) and the weight block as Bᵀ ([n][k]:
+// the BM x 64 activation tile (row-major) and the weight block as Bᵀ ([n][k]:
 // transposed while staging for the forward, as stored for dX) in LDS, rows
 // padded to 68 floats so the 16-byte reads of 16 consecutive rows hit all 64
 // banks once; the next entry's tiles are prefetched into registers during the
 // current entry's math. Wave w computes output rows 32w..32w+31 against both
-// 32-column halves. An MFMA step sums k = 4u + q (lanes 0-31) and 32 + 4u + q
+// 32-column halves (BM = 64: rows 32 (w % 2)..+31 against half w / 2). An MFMA step sums k = 4u + q (lanes 0-31) and 32 + 4u + q
 // (lanes 32-63), so each lane's operands for four steps are one 16-byte read
 // of its own row.
-constexpr int kBMf = 128;  // output rows per fp32 workgroup (4 waves x 32)
 constexpr int kPf = 68;    // LDS row pitch of the fp32 tiles, floats
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-template <bool FWD>
-__global__ __launch_bounds__(256, 2) void bell_gemm_f32_kernel(
+template <bool FWD, int BM>
+__global__ __launch_bounds__(256, BM == 64 ? 4 : 2) void bell_gemm_f32_kernel(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ vals,
     const int32_t* __restrict__ t_ptr, const int32_t* __restrict__ in_blk,
     const int32_t* __restrict__ t_vblk, const int32_t* __restrict__ order,
     const float* __restrict__ bias, int epi, float* __restrict__ Y, int64_t ldy,
     float* __restrict__ Z, int64_t ldz, int M, int n_out, int width, int n_mtiles, int per_xcd) {
-  __shared__ __attribute__((aligned(16))) float xs[kBMf * kPf];  // activation tile [m][k]
+  constexpr int XP = BM / 16;   // activation staging passes
+  constexpr int NC = BM / 64;   // 32-column halves per wave (BM = 64: waves split the columns)
+  __shared__ __attribute__((aligned(16))) float xs[BM * kPf];  // activation tile [m][k]
   __shared__ __attribute__((aligned(16))) float ws[64 * kPf];    // weight block as Bᵀ [n][k]
 
   const int logical = xcd_logical_id(per_xcd);
@@ -1092,22 +1093,24 @@ __global__ __launch_bounds__(256, 2) void bell_gemm_f32_kernel(
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int l32 = lane & 31, h = lane >> 5;
-  const int m0 = mtile * kBMf;
+  const int m0 = mtile * BM;
+  // wave: rows 32 wrow..+31 against the 32-column halves wcol..wcol + NC - 1
+  const int wrow = BM == 64 ? wave & 1 : wave, wcol = BM == 64 ? wave >> 1 : 0;
 
-  // Staging: activation rows 16p + tid/16 (p = 0..7), 16-byte chunk tid % 16 (16
+  // Staging: activation rows 16p + tid/16, 16-byte chunk tid % 16 (16
   // threads per 256-byte row); weight block: dX rows 16p + tid/16 as they are,
   // forward rows kk = tid % 64 with chunk tid/64 + 4p, written transposed.
   const int srow = tid >> 4, schunk = tid & 15;
-  int64_t xoff[8];
+  int64_t xoff[XP];
 #pragma unroll
-  for (int p = 0; p < 8; ++p)
+  for (int p = 0; p < XP; ++p)
     xoff[p] = static_cast<int64_t>(min(m0 + 16 * p + srow, M - 1)) * lda + 4 * schunk;
-  f32x4 px[8], pw[4];
+  f32x4 px[XP], pw[4];
   auto gload = [&](int e) __attribute__((always_inline)) {
     const float* xb = A + static_cast<int64_t>(in_blk[e]) * 64;
     const float* wb = vals + static_cast<int64_t>(FWD ? t_vblk[e] : e) * 4096;
 #pragma unroll
-    for (int p = 0; p < 8; ++p) px[p] = *reinterpret_cast<const f32x4*>(xb + xoff[p]);
+    for (int p = 0; p < XP; ++p) px[p] = *reinterpret_cast<const f32x4*>(xb + xoff[p]);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       if constexpr (FWD)
@@ -1118,7 +1121,7 @@ __global__ __launch_bounds__(256, 2) void bell_gemm_f32_kernel(
   };
   auto sstore = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < 8; ++p)
+    for (int p = 0; p < XP; ++p)
       *reinterpret_cast<f32x4*>(xs + (16 * p + srow) * kPf + 4 * schunk) = px[p];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -1134,13 +1137,12 @@ __global__ __launch_bounds__(256, 2) void bell_gemm_f32_kernel(
     }
   };
 
-  f32x16 acc[2];
-  acc[0] = f32x16{};
-  acc[1] = f32x16{};
+  f32x16 acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = f32x16{};
   if (e0 < e1) gload(e0);
-  const float* xa = xs + (32 * wave + l32) * kPf + 32 * h;
-  const float* wa0 = ws + l32 * kPf + 32 * h;
-  const float* wa1 = ws + (32 + l32) * kPf + 32 * h;
+  const float* xa = xs + (32 * wrow + l32) * kPf + 32 * h;
+  const float* wa = ws + (32 * wcol + l32) * kPf + 32 * h;
   for (int e = e0; e < e1; ++e) {
     __syncthreads();  // the previous entry's reads of xs / ws are done
     sstore();
@@ -1149,27 +1151,24 @@ __global__ __launch_bounds__(256, 2) void bell_gemm_f32_kernel(
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const f32x4 a = *reinterpret_cast<const f32x4*>(xa + 4 * u);
-      const f32x4 b0 = *reinterpret_cast<const f32x4*>(wa0 + 4 * u);
-      const f32x4 b1 = *reinterpret_cast<const f32x4*>(wa1 + 4 * u);
-      acc[0] = mfma_f32(a.x, b0.x, acc[0]);
-      acc[1] = mfma_f32(a.x, b1.x, acc[1]);
-      acc[0] = mfma_f32(a.y, b0.y, acc[0]);
-      acc[1] = mfma_f32(a.y, b1.y, acc[1]);
-      acc[0] = mfma_f32(a.z, b0.z, acc[0]);
-      acc[1] = mfma_f32(a.z, b1.z, acc[1]);
-      acc[0] = mfma_f32(a.w, b0.w, acc[0]);
-      acc[1] = mfma_f32(a.w, b1.w, acc[1]);
+      f32x4 bv[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) bv[c] = *reinterpret_cast<const f32x4*>(wa + 32 * c * kPf + 4 * u);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] = mfma_f32(a[t], bv[c][t], acc[c]);
     }
   }
 
-  // acc[ct][j] = out[m0 + 32w + 8(j/4) + 4h + j%4][64 ob + 32 ct + l32]
+  // acc[ct][j] = out[m0 + 32 wrow + 8(j/4) + 4h + j%4][64 ob + 32 (wcol + ct) + l32]
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const int col = 64 * ob + 32 * ct + l32;
+  for (int ct = 0; ct < NC; ++ct) {
+    const int col = 64 * ob + 32 * (wcol + ct) + l32;
     const float bv = bias ? bias[col] : 0.f;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      const int row = m0 + 32 * wave + 8 * (j >> 2) + 4 * h + (j & 3);
+      const int row = m0 + 32 * wrow + 8 * (j >> 2) + 4 * h + (j & 3);
       if (row >= M) continue;
       float v = acc[ct][j] + bv;
       if (Z) Z[static_cast<int64_t>(row) * ldz + col] = v;  // pre-activation (training)
@@ -1444,6 +1443,14 @@ int launch_status() {
   return err == hipSuccess ? TMAC_OK : static_cast<int>(err);
 }
 
+// Output rows per workgroup of the fp32 gather GEMM. A 128-row tile reads less per product, a 64-row
+// one (waves split its columns) gives twice the workgroups, four to a CU: below 2048 tiles of 128 rows
+// (eight per CU) the smaller one is faster: 2049 rows 640 -> 2560 at 50 %, 61 -> 56 us forward and 56 ->
+// 49 dX, 2560 -> 640 76 -> 63 and 45 -> 43, 500 rows 70 -> 39 us; at 8192 rows (2560 tiles) both take 153 us.
+int f32_rows(int M, int n_out) {
+  return static_cast<int64_t>((M + 127) / 128) * n_out < 2048 ? 64 : 128;
+}
+
 // Split of the SDDMM reduction over M, rows per split a multiple of 64. The
 // 16-bit kernel (two workgroups per CU) takes as many splits as fit the 512
 // slots of one wave of workgroups, so no workgroup waits for a second round;
@@ -1491,15 +1498,21 @@ int bell_fwd_impl(const void* d_X, int64_t ldx, const void* d_vals, const int32_
   if (d_bias && !aligned16(d_bias)) return TMAC_ERR_ALIGN;
   if (d_Z && (!aligned16(d_Z) || (ldz % vec))) return TMAC_ERR_ALIGN;
   if (dtype == TMAC_F32) {
-    const int n_mt = (M + kBMf - 1) / kBMf;
+    const int bm = f32_rows(M, n_bcol), n_mt = (M + bm - 1) / bm;
     const int64_t tot = static_cast<int64_t>(n_mt) * n_bcol;
     if (tot > (1ll << 30)) return TMAC_ERR_SHAPE;
     const int pxcd = static_cast<int>((tot + 7) / 8);
-    hipLaunchKernelGGL((bell_gemm_f32_kernel<true>), dim3(8 * pxcd), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const float*>(d_X), ldx,
-                       static_cast<const float*>(d_vals), d_t_ptr, d_t_row, d_t_vblk, d_order,
-                       static_cast<const float*>(d_bias), epi, static_cast<float*>(d_Y), ldy,
-                       static_cast<float*>(d_Z), ldz, M, n_bcol, width, n_mt, pxcd);
+#define TMAC_F32_LAUNCH(BM)                                                                          \
+    hipLaunchKernelGGL((bell_gemm_f32_kernel<true, BM>), dim3(8 * pxcd), dim3(256), 0,              \
+                       static_cast<hipStream_t>(stream), static_cast<const float*>(d_X), ldx,       \
+                       static_cast<const float*>(d_vals), d_t_ptr, d_t_row, d_t_vblk, d_order,      \
+                       static_cast<const float*>(d_bias), epi, static_cast<float*>(d_Y), ldy,       \
+                       static_cast<float*>(d_Z), ldz, M, n_bcol, width, n_mt, pxcd)
+    if (bm == 64)
+      TMAC_F32_LAUNCH(64);
+    else
+      TMAC_F32_LAUNCH(128);
+#undef TMAC_F32_LAUNCH
     return launch_status();
   }
   const int n_mtiles = (M + kBM - 1) / kBM;
@@ -1657,15 +1670,21 @@ extern "C" int tmac_bell_dx(const void* d_dY, int64_t lddy, const void* d_vals,
   if (!aligned16(d_dY) || !aligned16(d_vals) || !aligned16(d_dX) || (lddy % vec) || (lddx % vec))
     return TMAC_ERR_ALIGN;
   if (dtype == TMAC_F32) {
-    const int n_mt = (M + kBMf - 1) / kBMf;
+    const int bm = f32_rows(M, n_brow), n_mt = (M + bm - 1) / bm;
     const int64_t tot = static_cast<int64_t>(n_mt) * n_brow;
     if (tot > (1ll << 30)) return TMAC_ERR_SHAPE;
     const int pxcd = static_cast<int>((tot + 7) / 8);
-    hipLaunchKernelGGL((bell_gemm_f32_kernel<false>), dim3(8 * pxcd), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const float*>(d_dY), lddy,
-                       static_cast<const float*>(d_vals), nullptr, d_col_idx, nullptr, nullptr,
-                       nullptr, 0, static_cast<float*>(d_dX), lddx, nullptr, 0, M, n_brow, width,
-                       n_mt, pxcd);
+#define TMAC_F32_LAUNCH(BM)                                                                          \
+    hipLaunchKernelGGL((bell_gemm_f32_kernel<false, BM>), dim3(8 * pxcd), dim3(256), 0,             \
+                       static_cast<hipStream_t>(stream), static_cast<const float*>(d_dY), lddy,     \
+                       static_cast<const float*>(d_vals), nullptr, d_col_idx, nullptr, nullptr,     \
+                       nullptr, 0, static_cast<float*>(d_dX), lddx, nullptr, 0, M, n_brow, width,   \
+                       n_mt, pxcd)
+    if (bm == 64)
+      TMAC_F32_LAUNCH(64);
+    else
+      TMAC_F32_LAUNCH(128);
+#undef TMAC_F32_LAUNCH
     return launch_status();
   }
   const int n_mtiles = (M + kBM - 1) / kBM;
