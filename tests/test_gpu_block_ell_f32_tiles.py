@@ -35,3 +35,24 @@ def test_f32_products(dev, M, n_brow, n_bcol, width):
     rows = torch.arange(n_brow, device=dev)[:, None]
     err = (dv.double() - ref[rows, ci.long()]).abs()
     assert torch.all(err <= (M + 2) * 2.0 ** -24 * mag[rows, ci.long()])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n_brow,n_bcol,width", [(40, 10, 5), (7, 4, 3), (16, 8, 6), (9, 16, 9), (1, 8, 5)])
+@pytest.mark.parametrize("M", [1, 33, 700, 2100])
+def test_sddmm_blocks_across_rows(dev, M, n_brow, n_bcol, width, dtype):
+    """Widths whose blocks are taken four at a time across block-rows: every block of dW, twice the same."""
+    g = torch.Generator().manual_seed(M + width)
+    pat = kb.BlockELLPattern.sample(3, n_brow, n_bcol, width)
+    x = torch.randn(M, 64 * n_brow, generator=g).to(dev, dtype)
+    gy = torch.randn(M, 64 * n_bcol, generator=g).to(dev, dtype)
+    ci = torch.from_numpy(pat.col_idx).to(dev)
+    dv = kb._bell_sddmm(x, gy, ci.reshape(-1), n_brow, width, torch.float32)
+    assert torch.equal(dv, kb._bell_sddmm(x, gy, ci.reshape(-1), n_brow, width, torch.float32))
+
+    def blocks(a, b):
+        full = (a.double().t() @ b.double()).reshape(n_brow, 64, n_bcol, 64).permute(0, 2, 1, 3)
+        return full[torch.arange(n_brow, device=dev)[:, None], ci.long()]
+    # fp32 sums of exact products in any order (16-bit) or of rounded ones (fp32)
+    err = (dv.double() - blocks(x, gy)).abs()
+    assert torch.all(err <= (M + 2) * 2.0 ** -24 * blocks(x.abs(), gy.abs()))

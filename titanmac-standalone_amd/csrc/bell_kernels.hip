@@ -915,53 +915,63 @@ __global__ __launch_bounds__(256) void bell_fwd_small_kernel(
   }
 }
 
-// s_waitcnt vmcnt(n) for n in {0, 5, 10}; the other counters are left alone.
-__device__ __forceinline__ void wait_vm(int n) {
-  if (n >= 10)
-    asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-  else if (n >= 5)
-    asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+// s_waitcnt vmcnt(later * CP), later = 0, 1 or 2; the other counters are left alone.
+template <int CP>
+__device__ __forceinline__ void wait_steps(int later) {
+  if (later >= 2)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CP) : "memory");
+  else if (later == 1)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CP) : "memory");
   else
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// Work of an SDDMM workgroup: four blocks, one per wave. NX = 1: four slots of one block-row (the
+// last group of a row whose width is not a multiple of 4 has idle waves). NX = 2 (sddmm_flat): blocks
+// 4i..4i+3 of all the rows' blocks in order, which at width >= 3 lie in at most two rows, so two X
+// tiles are copied per step and no wave idles.
 constexpr int kSdRows = 32;            // M rows per SDDMM step
-constexpr int kSdStages = 4;           // LDS ring depth (three steps of copies in flight)
 constexpr int kSdTile = kSdRows * 64;  // one 32x64 tile, 16-bit elements
-constexpr int kSdStage = 5 * kSdTile;  // X tile + four dY tiles (20 KB)
 
-template <int DT>
+template <int DT, int NX>
 __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
     const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ dY, int64_t lddy,
     const int32_t* __restrict__ col_idx, float* __restrict__ part, int M, int n_brow, int width,
     int n_sgroups, int rows_per_split, int n_splits, int per_xcd) {
-  // Ring of four stages; stage = X[m:m+32, 64r:+64] then dY[m:m+32, 64c_w:+64]
+  // Ring of stages; stage = NX tiles X[m:m+32, 64r:+64] then dY[m:m+32, 64c_w:+64]
   // for w = 0..3, each tile 32 rows of 64 elements, chunks swizzled as swz64.
+  constexpr int kSdStages = NX == 1 ? 4 : 3;    // 80 or 72 KB: two workgroups per CU
+  constexpr int kSdStage = (NX + 4) * kSdTile;  // 20 or 24 KB
+  constexpr int kCp = NX + 4;                   // copies per wave and step
   __shared__ __attribute__((aligned(16))) uint16_t ring[kSdStages * kSdStage];
 
-  const int per_split = n_brow * n_sgroups;
+  const int n_blocks = n_brow * width;
+  const int per_split = NX == 1 ? n_brow * n_sgroups : (n_blocks + 3) / 4;
   const int logical = xcd_logical_id(per_xcd);
   if (logical >= n_splits * per_split) return;
   const int split = logical / per_split;
   const int rem = logical - split * per_split;
-  const int r = rem / n_sgroups;
-  const int sg = rem - r * n_sgroups;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int h = lane >> 5, grp = (lane >> 4) & 1, l32 = lane & 31;
-  const int s = sg * 4 + wave;
-  const bool active = s < width;
-  // this wave's block-column; a slot past the row's width repeats the last one
-  // (copied, never used)
-  const int cw = col_idx[r * width + min(s, width - 1)];
+  // first block-row, this wave's block (one past the row's or the matrix's end repeats the last
+  // one: copied, never used) and its X tile
+  const int r = NX == 1 ? rem / n_sgroups : 4 * rem / width;
+  const int s = NX == 1 ? (rem - r * n_sgroups) * 4 + wave : 0;
+  const int blk0 = NX == 1 ? r * width + s : 4 * rem + wave;
+  const bool active = NX == 1 ? s < width : blk0 < n_blocks;
+  const int blk = NX == 1 ? r * width + min(s, width - 1) : min(blk0, n_blocks - 1);
+  const int r_last = NX == 1 ? r : min(4 * rem + 3, n_blocks - 1) / width;
+  const int xt_own = NX == 1 || blk / width == r ? 0 : 1;
+  const int cw = col_idx[blk];
 
   const int m_begin = split * rows_per_split;
   const int m_end = min(M, m_begin + rows_per_split);
   const int n_steps = (m_end - m_begin + kSdRows - 1) / kSdRows;
 
   // Copies per step and wave: its own dY tile (four 8-row instructions) and
-  // rows 8w..8w+7 of the X tile. Lane L of an instruction covering rows
+  // rows 8w..8w+7 of the X tiles. Lane L of an instruction covering rows
   // R..R+7 fills chunk position L & 7 of row R + L / 8 and fetches the global
   // chunk the swizzle stores there; the eight lanes of a row read 128
   // contiguous bytes. A lane's byte offsets from the step's first row are the
@@ -973,7 +983,9 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
     return pos ^ (((a & 1) << 2) | (a >> 1));
   };
   const int xrow = 8 * wave + drow;
-  const uint32_t xcol = 2u * (64 * r + 8 * swz_chunk(xrow, dpos));
+  uint32_t xcol[NX];
+#pragma unroll
+  for (int x = 0; x < NX; ++x) xcol[x] = 2u * (64 * (x ? r_last : r) + 8 * swz_chunk(xrow, dpos));
   uint32_t ycol[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) ycol[j] = 2u * (64 * cw + 8 * swz_chunk(8 * j + drow, dpos));
@@ -984,12 +996,14 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
     const uint16_t* xb = X + static_cast<int64_t>(m0) * ldx;
     const uint16_t* yb = dY + static_cast<int64_t>(m0) * lddy;
     const int lim = M - 1 - m0;  // rows beyond this one read it instead
-    dma_lds16(xb, static_cast<uint32_t>(min(xrow, lim)) * static_cast<uint32_t>(2 * ldx) + xcol,
-                 st + 8 * wave * 128);
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+      dma_lds16(xb, static_cast<uint32_t>(min(xrow, lim)) * static_cast<uint32_t>(2 * ldx) + xcol[x],
+                st + x * kSdTile * 2 + 8 * wave * 128);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       dma_lds16(yb, static_cast<uint32_t>(min(8 * j + drow, lim)) * static_cast<uint32_t>(2 * lddy) + ycol[j],
-                   st + (1 + wave) * kSdTile * 2 + 8 * j * 128);
+                   st + (NX + wave) * kSdTile * 2 + 8 * j * 128);
   };
 
   f32x16 acc[2][2];
@@ -1002,17 +1016,20 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
   for (int i = 0; i < n_steps; ++i) {
     // this wave's copies of step i have landed when at most those of the
     // (up to kSdStages - 2) later steps already issued are outstanding
-    wait_vm(5 * min(kSdStages - 2, n_steps - 1 - i));
+    wait_steps<kCp>(min(kSdStages - 2, n_steps - 1 - i));
     const int m0 = m_begin + i * kSdRows;
     uint16_t* st = ring + (i % kSdStages) * kSdStage;
     if (m0 + kSdRows > m_end) {
       // rows past the range contribute zero: each wave clears the rows it copied
       const int valid = m_end - m0;
-      if (xrow >= valid) sts16(st + xrow * 64 + 8 * dpos, u32x4{0u, 0u, 0u, 0u});
+      if (xrow >= valid) {
+#pragma unroll
+        for (int x = 0; x < NX; ++x) sts16(st + x * kSdTile + xrow * 64 + 8 * dpos, u32x4{0u, 0u, 0u, 0u});
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (8 * j + drow >= valid)
-          sts16(st + (1 + wave) * kSdTile + (8 * j + drow) * 64 + 8 * dpos, u32x4{0u, 0u, 0u, 0u});
+          sts16(st + (NX + wave) * kSdTile + (8 * j + drow) * 64 + 8 * dpos, u32x4{0u, 0u, 0u, 0u});
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     // every wave's copies of step i are in LDS, and every wave is done reading
@@ -1020,8 +1037,8 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
     asm volatile("s_barrier" ::: "memory");
     if (i + kSdStages - 1 < n_steps) issue(i + kSdStages - 1);
     if (active) {
-      const uint16_t* xt = st;
-      const uint16_t* dyt = st + (1 + wave) * kSdTile;
+      const uint16_t* xt = st + xt_own * kSdTile;
+      const uint16_t* dyt = st + (NX + wave) * kSdTile;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         u32x4 af[2], bf[2];
@@ -1038,7 +1055,7 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
   }
 
   if (!active) return;
-  float* dst = part + (static_cast<int64_t>(split) * n_brow * width + r * width + s) * 4096;
+  float* dst = part + (static_cast<int64_t>(split) * n_blocks + blk) * 4096;
 #pragma unroll
   for (int ki = 0; ki < 2; ++ki)
 #pragma unroll
@@ -1184,41 +1201,50 @@ __global__ __launch_bounds__(256, BM == 64 ? 4 : 2) void bell_gemm_f32_kernel(
 // in LDS (rows past the range are zero); the wave's 64x64 block is four 32x32
 // MFMA tiles, an MFMA step summing rows m + 2s (lanes 0-31) and m + 2s + 1
 // (lanes 32-63). Partial sums go to the workspace as in the 16-bit kernel.
+template <int NX>
 __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
     const float* __restrict__ X, int64_t ldx, const float* __restrict__ dY, int64_t lddy,
     const int32_t* __restrict__ col_idx, float* __restrict__ part, int M, int n_brow, int width,
     int n_sgroups, int rows_per_split, int n_splits, int per_xcd) {
-  __shared__ __attribute__((aligned(16))) float xs[32 * 64];
+  __shared__ __attribute__((aligned(16))) float xs[NX][32 * 64];
   __shared__ __attribute__((aligned(16))) float ds[4][32 * 64];
 
-  const int per_split = n_brow * n_sgroups;
+  const int n_blocks = n_brow * width;
+  const int per_split = NX == 1 ? n_brow * n_sgroups : (n_blocks + 3) / 4;
   const int logical = xcd_logical_id(per_xcd);
   if (logical >= n_splits * per_split) return;
   const int split = logical / per_split;
   const int rem = logical - split * per_split;
-  const int r = rem / n_sgroups;
-  const int sg = rem - r * n_sgroups;
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int l32 = lane & 31, h = lane >> 5;
-  const int s = sg * 4 + wave;
-  const bool active = s < width;
-  const int c = col_idx[r * width + min(s, width - 1)];  // inactive waves stage a valid tile
+  // as in bell_sddmm_kernel; inactive waves stage a valid tile
+  const int r = NX == 1 ? rem / n_sgroups : 4 * rem / width;
+  const int s = NX == 1 ? (rem - r * n_sgroups) * 4 + wave : 0;
+  const int blk0 = NX == 1 ? r * width + s : 4 * rem + wave;
+  const bool active = NX == 1 ? s < width : blk0 < n_blocks;
+  const int blk = NX == 1 ? r * width + min(s, width - 1) : min(blk0, n_blocks - 1);
+  const int r_last = NX == 1 ? r : min(4 * rem + 3, n_blocks - 1) / width;
+  const int xt_own = NX == 1 || blk / width == r ? 0 : 1;
+  const int c = col_idx[blk];
   const int m_lo = split * rows_per_split;
   const int m_hi = min(M, m_lo + rows_per_split);
 
   // X: rows tid/16 and 16 + tid/16, chunk tid % 16; dY: the wave's lanes, rows
   // 4p + lane/16 (p = 0..7), chunk lane % 16.
   const int xr = tid >> 4, xc = tid & 15, dr = lane >> 4, dc = lane & 15;
-  f32x4 px[2], pd[8];
+  f32x4 px[NX][2], pd[8];
   auto gload = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       const int row = m + 16 * p + xr;
-      const f32x4 v = *reinterpret_cast<const f32x4*>(
-          X + static_cast<int64_t>(min(row, M - 1)) * ldx + 64 * r + 4 * xc);
-      px[p] = row < m_hi ? v : f32x4{};
+#pragma unroll
+      for (int x = 0; x < NX; ++x) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(
+            X + static_cast<int64_t>(min(row, M - 1)) * ldx + 64 * (x ? r_last : r) + 4 * xc);
+        px[x][p] = row < m_hi ? v : f32x4{};
+      }
     }
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
@@ -1228,17 +1254,30 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
   };
   auto sstore = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p) *reinterpret_cast<f32x4*>(xs + (16 * p + xr) * 64 + 4 * xc) = px[p];
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int x = 0; x < NX; ++x) *reinterpret_cast<f32x4*>(xs[x] + (16 * p + xr) * 64 + 4 * xc) = px[x][p];
 #pragma unroll
     for (int p = 0; p < 8; ++p)
       *reinterpret_cast<f32x4*>(ds[wave] + (4 * p + dr) * 64 + 4 * dc) = pd[p];
   };
 
-  f32x16 acc[2][2];
+  // Sums of 128 rows, added to the running ones: short chains, so that a long range is summed as
+  // exactly as many short ones.
+  f32x16 acc[2][2], tot[2][2];
+  auto flush = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        tot[a][b] += acc[a][b];
+        acc[a][b] = f32x16{};
+      }
+  };
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x16{};
+    for (int b = 0; b < 2; ++b) acc[a][b] = tot[a][b] = f32x16{};
   if (m_lo < m_hi) gload(m_lo);
   for (int m = m_lo; m < m_hi; m += 32) {
     __syncthreads();
@@ -1246,20 +1285,23 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
     __syncthreads();
     if (m + 32 < m_hi) gload(m + 32);
     const float* dsw = ds[wave];
+    const float* xsw = xs[xt_own];
 #pragma unroll
     for (int st = 0; st < 16; ++st) {
       const int row = 2 * st + h;
-      const float a0 = xs[row * 64 + l32], a1 = xs[row * 64 + 32 + l32];
+      const float a0 = xsw[row * 64 + l32], a1 = xsw[row * 64 + 32 + l32];
       const float b0 = dsw[row * 64 + l32], b1 = dsw[row * 64 + 32 + l32];
       acc[0][0] = mfma_f32(a0, b0, acc[0][0]);
       acc[0][1] = mfma_f32(a0, b1, acc[0][1]);
       acc[1][0] = mfma_f32(a1, b0, acc[1][0]);
       acc[1][1] = mfma_f32(a1, b1, acc[1][1]);
     }
+    if (((m - m_lo) & 96) == 96) flush();
   }
+  flush();
 
   if (!active) return;
-  float* dst = part + (static_cast<int64_t>(split) * n_brow * width + r * width + s) * 4096;
+  float* dst = part + (static_cast<int64_t>(split) * n_blocks + blk) * 4096;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -1267,7 +1309,7 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int kk = 32 * a + 8 * (j >> 2) + 4 * h + (j & 3);
-        dst[kk * 64 + 32 * b + l32] = acc[a][b][j];
+        dst[kk * 64 + 32 * b + l32] = tot[a][b][j];
       }
 }
 
@@ -1451,20 +1493,41 @@ int f32_rows(int M, int n_out) {
   return static_cast<int64_t>((M + 127) / 128) * n_out < 2048 ? 64 : 128;
 }
 
-// Split of the SDDMM reduction over M, rows per split a multiple of 64. The
-// 16-bit kernel (two workgroups per CU) takes as many splits as fit the 512
-// slots of one wave of workgroups, so no workgroup waits for a second round;
-// the fp32 kernel (four per CU) about 512 workgroups or a few more.
+// Whether the SDDMM takes the rows' blocks four at a time across rows (NX = 2): with groups of one
+// row's slots the last group of a width that is not a multiple of 4 has idle waves. The second X tile
+// makes a step's copies 24 KB instead of 20, so it pays where it saves more than a fifth of the
+// workgroups: widths 3, 5, 6, 9. Width 5, 2560 -> 640 at 50 %: bf16 32768 rows 92 -> 81 us, fp32 2049 rows 78 -> 56, 8192 rows 252 -> 172.
+bool sddmm_flat(int n_brow, int width) {
+  const int64_t rows = static_cast<int64_t>(n_brow) * ((width + 3) / 4);
+  return width >= 3 && (static_cast<int64_t>(n_brow) * width + 3) / 4 * 6 < rows * 5;
+}
+int sddmm_groups(int n_brow, int width) {
+  return sddmm_flat(n_brow, width) ? (n_brow * width + 3) / 4 : n_brow * ((width + 3) / 4);
+}
+
+// Split of the SDDMM reduction over M, rows per split a multiple of 64: the cheapest of a model of its
+// time in microseconds. A CU that holds L workgroups takes a 64-row step of each in 0.7 L us (16 bit;
+// 1.05 alone) or 3.9 L + 0.3 (fp32, bound by its MFMAs; 5.2 alone); the partial sums are written and
+// read once at about 4.5 TB/s. (Filling 512 workgroup slots whatever M is wrote 8-11 partial copies of dW for a few
+// steps each: fp32 2049 x 640 -> 2560 55 -> 48 us, 2560 -> 640 56 -> 49, bf16 1000 x 640 -> 2560 22.5 -> 18.3.)
 void sddmm_split(int M, int n_brow, int width, bool f32, int* n_splits, int* rows_per_split) {
-  const int n_sg = (width + 3) / 4;
-  const int base = n_brow * n_sg;
+  const int base = sddmm_groups(n_brow, width);
   const int m_steps = (M + 63) / 64;
-  int want = f32 ? (512 + base - 1) / base : 512 / base;
-  if (want < 1) want = 1;
-  if (want > m_steps) want = m_steps;
-  const int steps_per = (m_steps + want - 1) / want;
-  *rows_per_split = steps_per * 64;
-  *n_splits = (M + *rows_per_split - 1) / *rows_per_split;
+  const float part_us = static_cast<float>(n_brow) * width * 16384.f * 2.f / 4.5e6f;
+  float best_us = 0.f;
+  const int most = 1024 / base > 1 ? 1024 / base : 1;  // up to four workgroups per CU
+  for (int want = 1; want <= most && want <= m_steps; ++want) {
+    const int steps = (m_steps + want - 1) / want;
+    const int n = (m_steps + steps - 1) / steps;
+    const int64_t load = (static_cast<int64_t>(n) * base + 255) / 256;
+    const float step_us = f32 ? (load == 1 ? 5.2f : 3.9f * load + 0.3f) : (load == 1 ? 1.05f : 0.7f * load);
+    const float us = steps * step_us + n * part_us;
+    if (want == 1 || us < best_us) {
+      best_us = us;
+      *n_splits = n;
+      *rows_per_split = steps * 64;
+    }
+  }
 }
 
 // Workspace of tmac_bell_sddmm: the partial sums of the larger of the two
@@ -1786,24 +1849,32 @@ extern "C" int tmac_bell_sddmm(const void* d_X, int64_t ldx, const void* d_dY, i
   // the 16-bit kernel addresses 32 rows of X and dY with 32-bit byte offsets
   if (dtype != TMAC_F32 && (ldx > (1ll << 25) || lddy > (1ll << 25))) return TMAC_ERR_SHAPE;
   const int n_sg = (width + 3) / 4;
-  const int64_t total = static_cast<int64_t>(n_splits) * n_brow * n_sg;
+  const int64_t total = static_cast<int64_t>(n_splits) * sddmm_groups(n_brow, width);
   const int per_xcd = static_cast<int>((total + 7) / 8);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto* X = static_cast<const uint16_t*>(d_X);
   const auto* dY = static_cast<const uint16_t*>(d_dY);
   float* part = static_cast<float*>(d_ws);
-  if (dtype == TMAC_F32)
-    hipLaunchKernelGGL(bell_sddmm_f32_kernel, dim3(8 * per_xcd), dim3(256), 0, s,
-                       static_cast<const float*>(d_X), ldx, static_cast<const float*>(d_dY), lddy,
-                       d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits, per_xcd);
-  else if (dtype == TMAC_BF16)
-    hipLaunchKernelGGL((bell_sddmm_kernel<TMAC_BF16>), dim3(8 * per_xcd), dim3(256), 0, s, X, ldx,
-                       dY, lddy, d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits,
-                       per_xcd);
+#define TMAC_SDDMM_LAUNCH(NX)                                                                              \
+  do {                                                                                                     \
+    if (dtype == TMAC_F32)                                                                                 \
+      hipLaunchKernelGGL(bell_sddmm_f32_kernel<NX>, dim3(8 * per_xcd), dim3(256), 0, s,                    \
+                         static_cast<const float*>(d_X), ldx, static_cast<const float*>(d_dY), lddy,       \
+                         d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits, per_xcd);      \
+    else if (dtype == TMAC_BF16)                                                                           \
+      hipLaunchKernelGGL((bell_sddmm_kernel<TMAC_BF16, NX>), dim3(8 * per_xcd), dim3(256), 0, s, X, ldx,   \
+                         dY, lddy, d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits,      \
+                         per_xcd);                                                                         \
+    else                                                                                                   \
+      hipLaunchKernelGGL((bell_sddmm_kernel<TMAC_F16, NX>), dim3(8 * per_xcd), dim3(256), 0, s, X, ldx,    \
+                         dY, lddy, d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits,      \
+                         per_xcd);                                                                         \
+  } while (0)
+  if (sddmm_flat(n_brow, width))
+    TMAC_SDDMM_LAUNCH(2);
   else
-    hipLaunchKernelGGL((bell_sddmm_kernel<TMAC_F16>), dim3(8 * per_xcd), dim3(256), 0, s, X, ldx,
-                       dY, lddy, d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits,
-                       per_xcd);
+    TMAC_SDDMM_LAUNCH(1);
+#undef TMAC_SDDMM_LAUNCH
   st = launch_status();
   if (st != TMAC_OK) return st;
   const int64_t n_elem = static_cast<int64_t>(n_brow) * width * 4096;

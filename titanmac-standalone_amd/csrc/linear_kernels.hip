@@ -404,7 +404,8 @@ WGradPlan wgrad_plan(int M, int N, int K) {
   const int m_steps = (M + 63) / 64;
   for (int rn = 2; rn <= 4; rn += 2) {
     const int n_nt = (N + 64 * rn - 1) / (64 * rn), n_kt = (K + 127) / 128;
-    for (int want = 1; want <= 64 && want <= m_steps; ++want) {
+    const int most = 256 / (n_nt * n_kt) > 64 ? 256 / (n_nt * n_kt) : 64;
+    for (int want = 1; want <= most && want <= m_steps; ++want) {
       const int steps = (m_steps + want - 1) / want;
       const int n_splits = (m_steps + steps - 1) / steps;
       const int rounds = (n_nt * n_kt * n_splits + 255) / 256;
