@@ -1935,6 +1935,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void wattn_bwd_kv_f32m_kernel(
 // 2. wattn_mask_compact_kernel: one wave per list row (query-major rows, then
 //    key-major rows): entries[row * n_t + c] = t | kinds << 16 for the tiles t
 //    with a nonzero kind, t ascending, and cnt[row] = their number.
+template <bool BOOL>
 __global__ __launch_bounds__(256) void wattn_mask_kinds_kernel(AttnX ax, int S, int n_b, int n_t,
                                                                uint8_t* __restrict__ kinds_q,
                                                                uint8_t* __restrict__ kinds_kv,
@@ -1950,11 +1951,46 @@ __global__ __launch_bounds__(256) void wattn_mask_kinds_kernel(AttnX ax, int S, 
   uint32_t col0 = 0, col1 = 0;    // this lane's keys: allowed bits of the 32 rows
   uint64_t row0 = 0, row1 = 0;    // lane r < 32: allowed bits of row r, key tiles 2j, 2j + 1
   const int k0 = j * 128 + lane, k1 = k0 + 64;
-#pragma unroll 8
+  // The loads of kB rows are in flight before their ballots (with a test of the format and the edges
+  // around each load they stood one latency after another): bool masks 16 rows, 15.6 -> 10.3 us at S =
+  // 1537 and 22.3 -> 16.6 at 4096; float masks, four times the bytes, 8 rows (16 rows cost occupancy:
+  // 21.4 -> 24.0 at 4096, now 22.8). Positions past S read the last row or key and count as masked.
+  constexpr int kB = BOOL ? 16 : 8;
+  const int64_t moff = (ax.mb1 ? 0 : static_cast<int64_t>(bm) * ax.msb) +
+                       (ax.mh1 ? 0 : static_cast<int64_t>(hm) * ax.msh);
+  const int q0 = i * 128 + 32 * wave;
+  const int kc0 = min(k0, S - 1), kc1 = min(k1, S - 1);
+  float v[2][kB];
+#pragma unroll
   for (int r = 0; r < 32; ++r) {
-    const int q = i * 128 + 32 * wave + r;
-    const float v0 = mask_bias(ax, bm, hm, q, k0, S);
-    const float v1 = mask_bias(ax, bm, hm, q, k1, S);
+    if (r % kB == 0) {
+      if constexpr (BOOL) {
+        const uint8_t* m = static_cast<const uint8_t*>(ax.mask) + moff;
+        uint8_t t[2][kB];
+#pragma unroll
+        for (int rr = 0; rr < kB; ++rr) {
+          const uint8_t* row = m + static_cast<int64_t>(min(q0 + r + rr, S - 1)) * ax.msq;
+          t[0][rr] = row[kc0];
+          t[1][rr] = row[kc1];
+        }
+#pragma unroll
+        for (int rr = 0; rr < kB; ++rr) {
+          v[0][rr] = t[0][rr] ? 0.f : -INFINITY;
+          v[1][rr] = t[1][rr] ? 0.f : -INFINITY;
+        }
+      } else {
+        const float* m = static_cast<const float*>(ax.mask) + moff;
+#pragma unroll
+        for (int rr = 0; rr < kB; ++rr) {
+          const float* row = m + static_cast<int64_t>(min(q0 + r + rr, S - 1)) * ax.msq;
+          v[0][rr] = row[kc0];
+          v[1][rr] = row[kc1];
+        }
+      }
+    }
+    const bool in = q0 + r < S;
+    const float v0 = in && k0 < S ? v[0][r % kB] : -INFINITY;
+    const float v1 = in && k1 < S ? v[1][r % kB] : -INFINITY;
     const bool a0 = !(v0 == -INFINITY), a1 = !(v1 == -INFINITY);
     any0 |= a0;
     all0 &= (v0 == 0.f);
@@ -2537,7 +2573,14 @@ extern "C" int tmac_wattn_mask_lists(const tmac_attn_opts* opts, int S, void* st
   char* ws = static_cast<char*>(opts->d_mask_ws);
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto* kinds_q = reinterpret_cast<uint8_t*>(ws + w.kinds_q);
-  hipLaunchKernelGGL(wattn_mask_kinds_kernel, dim3(n_b, n_b, static_cast<unsigned>(n_mr)),
+  if (x.fmt == TMAC_MASK_BOOL)
+    hipLaunchKernelGGL(wattn_mask_kinds_kernel<true>, dim3(n_b, n_b, static_cast<unsigned>(n_mr)),
+                     dim3(256), 0, s, x, S, n_b, n_t, kinds_q,
+                     reinterpret_cast<uint8_t*>(ws + w.kinds_kv),
+                     reinterpret_cast<uint64_t*>(ws + w.bits_q),
+                     reinterpret_cast<uint32_t*>(ws + w.bits_kv));
+  else
+    hipLaunchKernelGGL(wattn_mask_kinds_kernel<false>, dim3(n_b, n_b, static_cast<unsigned>(n_mr)),
                      dim3(256), 0, s, x, S, n_b, n_t, kinds_q,
                      reinterpret_cast<uint8_t*>(ws + w.kinds_kv),
                      reinterpret_cast<uint64_t*>(ws + w.bits_q),
