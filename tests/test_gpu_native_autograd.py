@@ -83,8 +83,9 @@ def test_eager_native_only_in_plain_eager_mode():
         assert not _lib.eager_native(t)
     got = []
     torch.func.vmap(lambda v: got.append(_lib.eager_native(t)) or v)(t)
+    torch.jit.trace(lambda v: got.append(_lib.eager_native(v)) or v + 1, t, check_trace=False)
     torch.func.grad(lambda v: got.append(_lib.eager_native(t)) or v.sum())(t)
-    assert got == [False, False]
+    assert got == [False, False, False]
 
     class Sub(torch.Tensor):
         pass

@@ -200,8 +200,9 @@ def direct_call(*tensors: torch.Tensor | None) -> bool:
 def eager_native(*tensors: torch.Tensor | None) -> bool:
     """Whether an op may record its autograd node with a plain autograd.Function and run its kernels
     directly: eager mode, plain tensors, and nothing that rewrites, traces or intercepts torch calls
-    (torch.compile, functorch transforms, forward-mode AD, function or dispatch modes)."""
-    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+    (torch.compile, torch.jit.trace, functorch transforms, forward-mode AD, function or dispatch modes)."""
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0
             or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()):
         return False
