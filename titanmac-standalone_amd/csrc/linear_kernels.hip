@@ -146,9 +146,9 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(
   const bool active = col0 < N;
   issue(0);
   for (int i = 0; i < n_steps; ++i) {
-    // every wave's copies of step i are in LDS, and every wave is done with step i - 1, whose stage
-    // the next copies overwrite
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // every wave's copies of step i are in LDS, and every wave is done with step i - 1 (its reads have
+    // returned), whose stage the next copies overwrite
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");
     if (i + 1 < n_steps) issue(i + 1);
     if (active) compute(smem + (i & 1) * kLStage);
@@ -274,10 +274,10 @@ __global__ __launch_bounds__(512, 1) void linear_wgrad_kernel(
 #pragma unroll
         for (int t = 0; t < G::kTiles; ++t) sts16(st + t * 2048 + crow * 64 + 8 * dpos, u32x4{0u, 0u, 0u, 0u});
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    // every wave's copies of step i are in LDS, and every wave is done with step i - 1, whose stage
-    // the next copies overwrite
+    // every wave's copies of step i are in LDS, and every wave is done with step i - 1 (its reads have
+    // returned), whose stage the next copies overwrite
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");
     if (i + G::kStages - 1 < n_steps) issue(i + G::kStages - 1);
 #pragma unroll

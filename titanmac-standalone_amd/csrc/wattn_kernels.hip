@@ -1155,6 +1155,7 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
       span = mask_col_span(mp, key);
       load_kv();
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");  // every wave is done with the ring
     const uint16_t* st = ring + wave * (kKvStageB / 2);
     float* lse2 = reinterpret_cast<float*>(const_cast<uint16_t*>(st) + 2 * (kKvTileB / 2));
@@ -1182,6 +1183,7 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
       lse2[64 + lane] = -lse2[64 + lane];
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       process(ent, st, lse2);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // its reads have returned: the stage is free
     }
     // The helpers' sums through LDS (lane-major), added in wave order.
     float* red = reinterpret_cast<float*>(ring);  // 3 x 64 x 64 floats
