@@ -10,7 +10,7 @@
 // so no transposes are needed.
 //
 // Memory-bound stencil: each thread owns one 16-byte vector of channels and a
-// chunk of 64 consecutive positions, keeps a window of input rows in registers
+// chunk of 8 to 64 consecutive positions (conv_chunk), keeps a window of input rows in registers
 // (fp32), loads the rows in groups of 4 before using them (four loads in
 // flight per thread) and writes each output row once; consecutive threads read
 // consecutive 16-byte pieces of a row, so every row is read with full
@@ -22,7 +22,6 @@ using namespace tmac;
 
 namespace {
 
-constexpr int kChunk = 64;  // positions per thread
 constexpr int kGroup = 4;   // rows loaded together before use (memory-level parallelism)
 
 template <int DT>
@@ -79,11 +78,28 @@ __device__ __forceinline__ void load_or_zero(const uint8_t* base, int64_t row_by
   for (int e = 0; e < NN; ++e) v[e] = ok ? v[e] : 0.f;
 }
 
+// Positions per thread. A chunk re-reads KS-1 halo rows and is walked in groups of kGroup rows one
+// after another, so short chunks are taken while the grid does not fill the chip (the walk sets the
+// time: 16 groups took 11 us whatever the size) and long ones where it does: forward up to nine waves per
+// CU, backward up to two (8 rows) or four, and up to 512 partial rows, which column_sum_kernel walks.
+// Forward / backward with the column sum, us, bf16, 1920 channels, 4 taps, 64-row chunks -> this rule:
+// 1 x 560 11.3 -> 3.5 / 25.3 -> 9.7, 8 x 560 13.7 -> 6.7 / 32.1 -> 20.8, 16 x 560 16.2 -> 12.8 / 34.4 ->
+// 27.0; 32 x 560 23.8 -> 22.8 / 43.1 (32 rows: 52.2); 8 x 4096 64 rows: 38.9 / 89.1 (32 rows: 39.5 / 94.6).
+// 600 partial rows: 32 x 600 x 768 backward 40.7 with 32 rows, 37.8 with 64. n: elements per 16-byte vector.
+int conv_chunk(int B, int T, int C, int ks, int n, bool bwd) {
+  for (int c = 8; c < 64; c *= 2) {
+    const int64_t rows = static_cast<int64_t>(B) * ((T + c - 1) / c);
+    const int64_t waves = (rows * (C / n) + 63) / 64;
+    if (c >= 2 * (ks - 1) && waves <= (!bwd ? 2304 : c == 8 ? 512 : 1100) && (!bwd || rows <= 512)) return c;
+  }
+  return 64;
+}
+
 template <int DT, int KS>
 __global__ __launch_bounds__(256) void dwconv_causal_kernel(const uint8_t* __restrict__ in,
                                                             int64_t ld_in, const uint8_t* __restrict__ w,
                                                             uint8_t* __restrict__ out, int64_t ld_out,
-                                                            int T, int C, int n_chunks) {
+                                                            int T, int C, int n_chunks, int chunk_len) {
   using V = Vec<DT>;
   constexpr int N = V::N;
   constexpr int E = DT == TMAC_F32 ? 4 : 2;  // bytes per element
@@ -91,8 +107,8 @@ __global__ __launch_bounds__(256) void dwconv_causal_kernel(const uint8_t* __res
   const int vc = blockIdx.y * 256 + threadIdx.x;
   if (vc * N >= C) return;
   const int b = blockIdx.x / n_chunks;
-  const int t0 = (blockIdx.x - b * n_chunks) * kChunk;
-  const int t1 = min(t0 + kChunk, T);
+  const int t0 = (blockIdx.x - b * n_chunks) * chunk_len;
+  const int t1 = min(t0 + chunk_len, T);
   const int c0 = vc * N;
 
   // Taps of this thread's channels: wt[j][i] = w[c0 + i][j] (weights are
@@ -150,7 +166,7 @@ int launch_dwconv(const void* d_in, int64_t ld_in, const void* d_w, void* d_out,
                   int B, int T, int C, int ks, hipStream_t s) {
   constexpr int N = Vec<DT>::N;
   const int n_vec = C / N;
-  const int n_chunks = (T + kChunk - 1) / kChunk;
+  const int chunk_len = conv_chunk(B, T, C, ks, N, false), n_chunks = (T + chunk_len - 1) / chunk_len;
   const int64_t gx = static_cast<int64_t>(B) * n_chunks;
   const int gy = (n_vec + 255) / 256;
   if (gx > (1ll << 31) - 1 || gy > 65535) return TMAC_ERR_SHAPE;
@@ -161,7 +177,7 @@ int launch_dwconv(const void* d_in, int64_t ld_in, const void* d_w, void* d_out,
 #define TMAC_DWCONV_CASE(KS)                                                                   \
   case KS:                                                                                     \
     hipLaunchKernelGGL((dwconv_causal_kernel<DT, KS>), grid, dim3(256), 0, s, in, ld_in, w, out, \
-                       ld_out, T, C, n_chunks);                                                \
+                       ld_out, T, C, n_chunks, chunk_len);                                       \
     break;
   switch (ks) {
     TMAC_DWCONV_CASE(1)
@@ -183,7 +199,7 @@ int launch_dwconv(const void* d_in, int64_t ld_in, const void* d_w, void* d_out,
 // Backward, one pass over d_out and the input:
 //   d_in[b, t, c] = Σ_j w[c, j] · d_out[b, t + (k-1) - j, c]   (d_out[b, >= T, c] = 0)
 //   dw[c, j]     = Σ_{b, t} d_out[b, t, c] · in[b, t - (k-1) + j, c]
-// Each thread owns one 16-byte vector of channels and a chunk of 64 positions,
+// Each thread owns one 16-byte vector of channels and a chunk of positions,
 // walks the chunk from its end in groups of 4 rows with register windows of
 // the d_out rows from t on and the input rows up to t, writes each d_in row
 // once and its chunk's partial dw (fp32, tap-major) to one workspace row.
@@ -193,7 +209,7 @@ template <int DT, int KS>
 __global__ __launch_bounds__(256) void dwconv_causal_bwd_kernel(
     const uint8_t* __restrict__ dout, int64_t ld_dout, const uint8_t* __restrict__ in,
     int64_t ld_in, const uint8_t* __restrict__ w, uint8_t* __restrict__ din, int64_t ld_din,
-    float* __restrict__ partial, int T, int C, int n_chunks) {
+    float* __restrict__ partial, int T, int C, int n_chunks, int chunk_len) {
   using V = Vec<DT>;
   constexpr int N = V::N;
   constexpr int E = DT == TMAC_F32 ? 4 : 2;
@@ -202,8 +218,8 @@ __global__ __launch_bounds__(256) void dwconv_causal_bwd_kernel(
   if (vc * N >= C) return;
   const int b = blockIdx.x / n_chunks;
   const int chunk = blockIdx.x - b * n_chunks;
-  const int t0 = chunk * kChunk;
-  const int t1 = min(t0 + kChunk, T);
+  const int t0 = chunk * chunk_len;
+  const int t1 = min(t0 + chunk_len, T);
   const int c0 = vc * N;
 
   float wt[KS][N];
@@ -291,7 +307,7 @@ int launch_dwconv_bwd(const void* d_dout, int64_t ld_dout, const void* d_in, int
                       int T, int C, int ks, hipStream_t s) {
   constexpr int N = Vec<DT>::N;
   const int n_vec = C / N;
-  const int n_chunks = (T + kChunk - 1) / kChunk;
+  const int chunk_len = conv_chunk(B, T, C, ks, N, true), n_chunks = (T + chunk_len - 1) / chunk_len;
   const int64_t gx = static_cast<int64_t>(B) * n_chunks;
   const int gy = (n_vec + 255) / 256;
   if (gx > (1ll << 31) - 1 || gy > 65535) return TMAC_ERR_SHAPE;
@@ -303,7 +319,7 @@ int launch_dwconv_bwd(const void* d_dout, int64_t ld_dout, const void* d_in, int
 #define TMAC_DWCONV_BWD_CASE(KS)                                                              \
   case KS:                                                                                    \
     hipLaunchKernelGGL((dwconv_causal_bwd_kernel<DT, KS>), grid, dim3(256), 0, s, g, ld_dout, \
-                       in, ld_in, w, din, ld_din, ws, T, C, n_chunks);                        \
+                       in, ld_in, w, din, ld_din, ws, T, C, n_chunks, chunk_len);             \
     break;
   switch (ks) {
     TMAC_DWCONV_BWD_CASE(1)
@@ -325,8 +341,10 @@ int launch_dwconv_bwd(const void* d_dout, int64_t ld_dout, const void* d_in, int
   return err == hipSuccess ? TMAC_OK : static_cast<int>(err);
 }
 
+// One size for every type: the 16-bit chunks are never longer than the fp32 ones.
 size_t dwconv_bwd_ws_bytes(int B, int T, int C, int ks) {
-  const int64_t n_chunks = (T + kChunk - 1) / kChunk;
+  const int chunk_len = conv_chunk(B, T, C, ks, 8, true);
+  const int64_t n_chunks = (T + chunk_len - 1) / chunk_len;
   return static_cast<size_t>(B) * n_chunks * C * ks * sizeof(float);
 }
 
