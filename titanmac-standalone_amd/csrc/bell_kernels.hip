@@ -637,7 +637,7 @@ __global__ __launch_bounds__(512 * R, 1) void bell_ggemm_kernel(
       wait_vm_upto31(i == 0 ? pending : 0);
       // every wave's copies of step i are in LDS, and every wave is done with
       // step i - 1, whose stage the next copies overwrite
-      asm volatile("s_barrier" ::: "memory");
+      ring_barrier();
       if (i + 1 < n_steps) issue(i + 1, gs + i + 1);
       if (own_vb(i) >= 0) compute(smem + ((gs + i) & 1) * kX, smem + 2 * kX + ((gs + i) & 1) * kW + mem * 4096);
     }
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(512 * R, 1) void bell_ggemm_kernel(
     }
     // every wave is done with the ring before the next tile's copies go in
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier();
     ++rnd;
     const int t_next = next_tile(rnd);
     const bool more = t_next >= 0;
@@ -1030,11 +1030,10 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_kernel(
       for (int j = 0; j < 4; ++j)
         if (8 * j + drow >= valid)
           sts16(st + (NX + wave) * kSdTile + (8 * j + drow) * 64 + 8 * dpos, u32x4{0u, 0u, 0u, 0u});
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     // every wave's copies of step i are in LDS, and every wave is done reading
     // the stage the next copies overwrite (step i-1's)
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier();
     if (i + kSdStages - 1 < n_steps) issue(i + kSdStages - 1);
     if (active) {
       const uint16_t* xt = st + xt_own * kSdTile;

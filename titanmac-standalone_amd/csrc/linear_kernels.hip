@@ -148,8 +148,8 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(
   for (int i = 0; i < n_steps; ++i) {
     // every wave's copies of step i are in LDS, and every wave is done with step i - 1 (its reads have
     // returned), whose stage the next copies overwrite
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ring_barrier();
     if (i + 1 < n_steps) issue(i + 1);
     if (active) compute(smem + (i & 1) * kLStage);
   }
@@ -277,8 +277,7 @@ __global__ __launch_bounds__(512, 1) void linear_wgrad_kernel(
     }
     // every wave's copies of step i are in LDS, and every wave is done with step i - 1 (its reads have
     // returned), whose stage the next copies overwrite
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier();
     if (i + G::kStages - 1 < n_steps) issue(i + G::kStages - 1);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {

@@ -185,6 +185,14 @@ __device__ __forceinline__ void dma_lds4(const void* base, uint32_t voff, uint32
                : "memory", "m0");
 }
 
+// Barrier between the steps of a ring of copied LDS stages. Each wave arrives with its LDS reads returned
+// (of the stage that the copies issued after the barrier overwrite) and its LDS writes done. s_barrier alone
+// waits for neither: the compiler waits for a read where its value is used, and may move that MFMA past the
+// barrier. Copies in flight (vmcnt) are the caller's to wait for.
+__device__ __forceinline__ void ring_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Workgroup id remapped so that consecutive logical ids run on the same XCD:
 // the hardware hands workgroup b to XCD b % 8, so logical = (b % 8) * per_xcd +
 // b / 8 keeps each XCD on one contiguous slice of the logical work order (and

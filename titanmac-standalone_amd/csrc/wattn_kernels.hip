@@ -1127,11 +1127,10 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
       // copy has landed)
       float* v = lse2 + 64 * (wave - 2) + lane;
       *v = wave == 2 ? lse_log2<CM>(*v) : -*v;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     // every wave's copies of tile i are in LDS (and converted), and every wave
     // is done reading the stage the next copies overwrite (tile i-1's)
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier();
     if (i + kKvStages - 1 < n_main) issue(i + kKvStages - 1);
     const int ent = entries[e0 + i];
     if constexpr (CM) {
@@ -1155,8 +1154,7 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
       span = mask_col_span(mp, key);
       load_kv();
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");  // every wave is done with the ring
+    ring_barrier();  // every wave is done with the ring
     const uint16_t* st = ring + wave * (kKvStageB / 2);
     float* lse2 = reinterpret_cast<float*>(const_cast<uint16_t*>(st) + 2 * (kKvTileB / 2));
     const uint32_t sb = ring0 + static_cast<uint32_t>(wave * kKvStageB);
@@ -1187,7 +1185,7 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     }
     // The helpers' sums through LDS (lane-major), added in wave order.
     float* red = reinterpret_cast<float*>(ring);  // 3 x 64 x 64 floats
-    asm volatile("s_barrier" ::: "memory");        // every wave is done with its stage
+    ring_barrier();                                // every wave is done with its stage
     if (wave >= n_sl) {
 #pragma unroll
       for (int dt = 0; dt < T::kDt; ++dt)
@@ -1401,7 +1399,7 @@ __global__ __launch_bounds__(256, RING ? 4 : (D > 64 ? 1 : 3)) void wattn_bwd_q_
       // this wave's copies of tile e have landed; after the barrier every wave's
       // have, and every wave is done with tile e - 1, whose buffer the next copies fill
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      asm volatile("s_barrier" ::: "memory");
+      ring_barrier();
       if (more) issue(entries[e + 1] & 0xffff, buf ^ 1);
     } else if (more) {
       gload(entries[e + 1] & 0xffff);
