@@ -67,6 +67,55 @@ def test_fused_step_partial_gradients(dev):
     assert half.fc1.values.grad is not None and half.fc2.bias.grad is not None
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("frozen", [(), ("fc1.values", "fc2.values", "x"), ("fc1.values", "fc1.bias", "fc2.values", "fc2.bias")])
+def test_second_derivatives_are_not_dropped(dev, frozen):
+    """create_graph: the same first gradients, and what is built on them raises or is right (fc2's bias
+    gradient is a sum of the incoming one), whatever else requires grad: no gradient counts as a constant."""
+    torch.manual_seed(1)
+    mlp = MLPBlock(128, 256, block_ell=True, density=0.5).to(dev, torch.bfloat16)
+    x = torch.randn(40, 128, device=dev).bfloat16().requires_grad_("x" not in frozen)
+    ts = {"x": x, **dict(mlp.named_parameters())}
+    for n in frozen:
+        ts[n].requires_grad_(False)
+    ts = {n: t for n, t in ts.items() if t.requires_grad}
+    want = torch.autograd.grad(mlp(x).sum(), list(ts.values()))
+    got = torch.autograd.grad(mlp(x).sum(), list(ts.values()), create_graph=True)
+    for (n, g), w in zip(zip(ts, got), want):
+        if n == "fc1.bias":  # the recorded route sums the rounded terms: 40 of them
+            assert torch.allclose(g.float(), w.float(), rtol=2.0 ** -7, atol=40 * 2.0 ** -8), n
+        else:
+            assert torch.equal(g, w), n
+        assert g.requires_grad == (n != "fc2.bias"), n
+        if g.requires_grad:
+            with pytest.raises(RuntimeError):
+                torch.autograd.grad(g.float().pow(2).sum(), list(ts.values()), retain_graph=True, allow_unused=True)
+    if "fc2.bias" in ts:
+        gy = torch.randn(40, 128, device=dev).bfloat16().requires_grad_()
+        (gb,) = torch.autograd.grad(mlp(x), ts["fc2.bias"], gy, create_graph=True)
+        c = torch.randn(128, device=dev).bfloat16()
+        (gg,) = torch.autograd.grad(gb, gy, c)
+        assert torch.equal(gg, c.expand(40, 128))
+
+
+@pytest.mark.gpu
+def test_second_derivatives_of_single_layers(dev):
+    """As above for the layers by themselves: a GELU layer whose only tracked input is its bias, and a
+    plain layer's bias gradient."""
+    torch.manual_seed(2)
+    fc1, fc2 = (kb.BlockELLLinear(i, o, density=0.5).to(dev, torch.bfloat16) for i, o in ((128, 256), (256, 128)))
+    fc1.values.requires_grad_(False)
+    x = torch.randn(9, 128, device=dev).bfloat16()
+    (g,) = torch.autograd.grad(fc1(x, activation="gelu").sum(), fc1.bias, create_graph=True)
+    assert g.requires_grad
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(g.sum(), fc1.bias)
+    gy = torch.randn(9, 128, device=dev).bfloat16().requires_grad_()
+    (gb,) = torch.autograd.grad(fc2(torch.randn(9, 256, device=dev).bfloat16()), fc2.bias, gy, create_graph=True)
+    (gg,) = torch.autograd.grad(gb.sum(), gy)
+    assert torch.equal(gg, torch.ones_like(gy))
+
+
 def test_dx_gelu_argument_errors():
     import ctypes
     L, p = _lib.lib(), 4096  # an aligned address; nothing is launched

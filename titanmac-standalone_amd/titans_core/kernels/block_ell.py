@@ -423,6 +423,40 @@ def _sddmm_workspace_bytes(L, M: int, n_brow: int, n_bcol: int, width: int) -> i
     return int(out.value)
 
 
+def _bias_grad(gy: torch.Tensor, direct: bool) -> torch.Tensor:
+    """Column sums of gy [..., N]: the kernel's fixed-order fp32 sums, or where the backward is itself
+    recorded torch's, which can be differentiated."""
+    g2 = gy.reshape(-1, gy.shape[-1])
+    if g2.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+        return g2.sum(0)
+    return _bell_bias_grad(g2) if direct else g2.sum(0, dtype=torch.float32)
+
+
+class _FirstOrder(torch.autograd.Function):
+    """A gradient whose own derivative is not implemented, recorded as a function of what it depends on:
+    differentiating it raises, where a gradient without a graph would count as a constant."""
+    generate_vmap_rule = True
+
+    @staticmethod
+    def forward(g, *deps):
+        return g.clone()
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        pass
+
+    @staticmethod
+    def backward(ctx, gg):
+        raise RuntimeError("the Block-ELL GELU layers have no second derivative")
+
+
+def _first_order(g: Optional[torch.Tensor], *deps: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """g, in a recorded backward (create_graph) as a _FirstOrder of deps."""
+    if g is None or not torch.is_grad_enabled():
+        return g
+    return _FirstOrder.apply(g.detach(), *(d for d in deps if d is not None))
+
+
 def _fwd_setup_context(ctx, inputs, output):
     x, values, col_idx, t_ptr, t_row, t_vblk, order, bias, gelu, _grp, _tord = inputs
     if gelu:
@@ -450,11 +484,7 @@ def _fwd_backward(ctx, gy):
         gv = (_bell_sddmm if direct else bell_sddmm)(x, gy.to(x.dtype), col_idx, n_brow, width,
                                                      values.dtype)
     if ctx.has_bias and ctx.needs_input_grad[7]:
-        g2 = gy.reshape(-1, gy.shape[-1])
-        if g2.dtype in (torch.bfloat16, torch.float16, torch.float32):
-            gb = _bell_bias_grad(g2).to(g2.dtype)  # fixed-order fp32 column sums
-        else:
-            gb = g2.sum(0)
+        gb = _bias_grad(gy, direct).to(gy.dtype)
     return gx, gv, None, None, None, None, None, gb, None, None, None
 
 
@@ -470,6 +500,7 @@ def _fwd_gelu_setup_context(ctx, inputs, output):
     ctx.n_bcol = int(t_ptr.shape[0]) - 1
     ctx.has_bias = bias is not None
     ctx.bias_dtype = bias.dtype if bias is not None else None
+    ctx.bias = bias  # for its place in the graph of a recorded backward; its values are not used
 
 
 def _fwd_gelu_backward(ctx, ga, _gz_unused):
@@ -489,6 +520,7 @@ def _fwd_gelu_backward(ctx, ga, _gz_unused):
         gv = (_bell_sddmm if direct else bell_sddmm)(x, gz, col_idx, n_brow, width, values.dtype)
     if want_b:
         gb = db.to(ctx.bias_dtype)
+    gx, gv, gb = (_first_order(g, ga, x, values, ctx.bias) for g in (gx, gv, gb))
     return gx, gv, None, None, None, None, None, gb, None, None
 
 
@@ -589,6 +621,7 @@ class _MLP(torch.autograd.Function):
         ctx.save_for_backward(x, v1, z, a, v2, i1["col_idx"], i2["col_idx"])
         ctx.n_bcol = (i1["t_ptr"].numel() - 1, i2["t_ptr"].numel() - 1)
         ctx.bias_dtypes = [None if b is None else b.dtype for b in (b1, b2)]
+        ctx.b1 = b1  # for its place in the graph of a recorded backward; its values are not used
         return y
 
     @staticmethod
@@ -609,10 +642,12 @@ class _MLP(torch.autograd.Function):
                 g1 = sddmm(x, gz, c1, v1.shape[0], v1.shape[1], v1.dtype)
             if need[2]:
                 gb1 = db.to(ctx.bias_dtypes[0])
+            gx, g1, gb1 = (_first_order(g, gy, x, v1, ctx.b1, v2) for g in (gx, g1, gb1))
         if need[3]:
             g2 = sddmm(a, gy, c2, v2.shape[0], v2.shape[1], v2.dtype)
+            g2 = _first_order(g2, gy, x, v1, ctx.b1)  # a is fc1's output
         if need[4]:
-            gb2 = _bell_bias_grad(gy.reshape(-1, gy.shape[-1])).to(ctx.bias_dtypes[1])
+            gb2 = _bias_grad(gy, direct).to(ctx.bias_dtypes[1])
         return gx, g1, gb1, g2, gb2, None, None
 
 
