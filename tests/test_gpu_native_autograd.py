@@ -51,6 +51,47 @@ def test_routes_agree(dev, name, dtype, monkeypatch):
         assert a.dtype == b.dtype and torch.equal(a, b)
 
 
+def _mlp(dev, dtype):
+    from titans_core.blocks.mlp import MLPBlock
+    torch.manual_seed(4)
+    m = MLPBlock(128, 256, block_ell=True, density=0.5).to(dev, dtype)
+    ps = dict(m.named_parameters())
+    return (lambda x, *p: torch.func.functional_call(m, dict(zip(ps, p)), (x,))), [(30, 128)] + [p.shape for p in ps.values()]
+
+
+def _projection():
+    from titans_core.kernels.linear import projection
+    return projection, [(12010, 192), (640, 192)]
+
+
+def _fused_qkv(dropout_p=0.0):
+    from titans_core.kernels.window_attn import windowed_attention_qkv
+    return (lambda qkv: windowed_attention_qkv(qkv, 2, 40, 4, dropout_p=dropout_p)), [(2, 90, 384)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", [*CASES, "mlp", "projection", "fused_qkv", "fused_qkv_dropout"])
+def test_batched_gradients(dev, name):
+    """is_grads_batched: the backward meets batched tensors; each row's gradients are those of a backward
+    by itself (up to the order of a bias gradient's sum)."""
+    fn, shapes = {"mlp": lambda: _mlp(dev, torch.bfloat16), "projection": _projection, "fused_qkv": _fused_qkv,
+                  "fused_qkv_dropout": lambda: _fused_qkv(0.25)}.get(name, lambda: CASES[name])()
+    g = torch.Generator().manual_seed(6)
+    xs = [(torch.randn(*s, generator=g) * 0.3).to(dev, torch.bfloat16).requires_grad_() for s in shapes]
+    y = fn(*xs)
+    gys = torch.randn(3, *y.shape, generator=g).to(dev, torch.bfloat16)
+    batched = torch.autograd.grad(y, xs, gys, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for b, w in zip(batched, torch.autograd.grad(y, xs, gys[i], retain_graph=True)):
+            if w.dim() == 1:  # fp32 sums of up to 90 terms, rounded or not, rounded to bfloat16
+                assert torch.allclose(b[i].float(), w.float(), rtol=2.0 ** -7, atol=90 * 2.0 ** -8), name
+            elif name == "projection":  # the library's product: fp32 sums in another order, then rounded
+                scale = w.float().abs().max()
+                assert torch.allclose(b[i].float(), w.float(), rtol=2.0 ** -7, atol=2.0 ** -10 * scale), name
+            else:
+                assert torch.equal(b[i], w), name
+
+
 @pytest.mark.gpu
 def test_changed_input_is_noticed(dev):
     """An input changed in place between forward and backward raises, as for the registered op."""

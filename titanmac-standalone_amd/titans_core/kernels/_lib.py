@@ -197,6 +197,13 @@ def direct_call(*tensors: torch.Tensor | None) -> bool:
     return True
 
 
+def direct_backward(grad: torch.Tensor, *tensors: torch.Tensor | None) -> bool:
+    """direct_call in a backward of the incoming gradient `grad`: with is_grads_batched or under functorch
+    that is a batched tensor, whose Python type is torch.Tensor's own and which has no address."""
+    return (direct_call(grad, *tensors) and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._functorch.is_legacy_batchedtensor(grad))
+
+
 def eager_native(*tensors: torch.Tensor | None) -> bool:
     """Whether an op may record its autograd node with a plain autograd.Function and run its kernels
     directly: eager mode, plain tensors, and nothing that rewrites, traces or intercepts torch calls

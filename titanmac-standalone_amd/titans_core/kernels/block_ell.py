@@ -435,15 +435,10 @@ def _bias_grad(gy: torch.Tensor, direct: bool) -> torch.Tensor:
 class _FirstOrder(torch.autograd.Function):
     """A gradient whose own derivative is not implemented, recorded as a function of what it depends on:
     differentiating it raises, where a gradient without a graph would count as a constant."""
-    generate_vmap_rule = True
 
     @staticmethod
-    def forward(g, *deps):
+    def forward(ctx, g, *deps):
         return g.clone()
-
-    @staticmethod
-    def setup_context(ctx, inputs, output):
-        pass
 
     @staticmethod
     def backward(ctx, gg):
@@ -477,7 +472,7 @@ def _fwd_backward(ctx, gy):
     x, values, col_idx = ctx.saved_tensors
     n_brow, width = int(values.shape[0]), int(values.shape[1])
     gx = gv = gb = None
-    direct = _lib.direct_call(gy, x, values)
+    direct = _lib.direct_backward(gy, x, values)
     if ctx.needs_input_grad[0]:
         gx = (_bell_dx if direct else bell_dx)(gy, values, col_idx, ctx.n_bcol).to(x.dtype)
     if ctx.needs_input_grad[1]:
@@ -511,7 +506,7 @@ def _fwd_gelu_backward(ctx, ga, _gz_unused):
     if ga is None:
         ga = torch.zeros_like(z)
     want_b = ctx.has_bias and ctx.needs_input_grad[7]
-    direct = _lib.direct_call(ga, x, values, z)
+    direct = _lib.direct_backward(ga, x, values, z)
     gz, db = (_bell_gelu_bwd if direct else bell_gelu_bwd)(ga, z, want_b)
     gx = gv = gb = None
     if ctx.needs_input_grad[0]:
@@ -628,7 +623,7 @@ class _MLP(torch.autograd.Function):
     def backward(ctx, gy):
         x, v1, z, a, v2, c1, c2 = ctx.saved_tensors
         need = ctx.needs_input_grad
-        direct = _lib.direct_call(gy, x, v1, v2)  # else the backward is itself recorded: registered ops
+        direct = _lib.direct_backward(gy, x, v1, v2)  # else recorded or batched: registered ops
         dx, sddmm = (_bell_dx, _bell_sddmm) if direct else (bell_dx, bell_sddmm)
         gx = g1 = gb1 = g2 = gb2 = None
         if need[0] or need[1] or need[2]:

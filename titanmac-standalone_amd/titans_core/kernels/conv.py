@@ -95,7 +95,7 @@ def _setup(ctx, inputs, output):
 
 def _backward(ctx, grad):
     x, weight = ctx.saved_tensors
-    op = _dwconv_causal_bwd if _lib.direct_call(grad, x, weight) else dwconv_causal_bwd
+    op = _dwconv_causal_bwd if _lib.direct_backward(grad, x, weight) else dwconv_causal_bwd
     dx, dw = op(grad, x, weight)
     return dx, dw.to(weight.dtype)
 

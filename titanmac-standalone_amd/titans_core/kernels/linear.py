@@ -113,7 +113,7 @@ class _Projection(torch.autograd.Function):
     def backward(ctx, gy):
         x, weight = ctx.saved_tensors
         gx = gw = None
-        if torch.is_grad_enabled() or not _lib.eager_native(gy, x, weight):
+        if torch.is_grad_enabled() or not _lib.direct_backward(gy, x, weight):
             if ctx.needs_input_grad[0]:
                 gx = gy @ weight
             if ctx.needs_input_grad[1]:

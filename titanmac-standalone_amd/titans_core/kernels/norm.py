@@ -98,7 +98,7 @@ def _setup(ctx, inputs, output):
 
 def _backward(ctx, grad_y, grad_rstd):
     x, scale, rstd = ctx.saved_tensors
-    op = _rmsnorm_bwd if _lib.direct_call(grad_y, x, scale) else rmsnorm_bwd
+    op = _rmsnorm_bwd if _lib.direct_backward(grad_y, x, scale) else rmsnorm_bwd
     dx, dscale = op(grad_y, x, scale, rstd)
     return dx, dscale.to(scale.dtype), None
 

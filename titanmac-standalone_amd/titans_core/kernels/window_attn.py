@@ -281,7 +281,7 @@ def _backward(ctx, grad_out, grad_lse):
         raise RuntimeError("window_attn_fwd was called with need_lse=False; its backward "
                            "needs the log-sum-exp (windowed_attention sets it under autograd)")
     q, k, v, out, lse = ctx.saved_tensors
-    op = _window_attn_bwd if _lib.direct_call(grad_out, q, k, v) else window_attn_bwd
+    op = _window_attn_bwd if _lib.direct_backward(grad_out, q, k, v) else window_attn_bwd
     dq, dk, dv = op(grad_out, q, k, v, out, lse, *ctx.args)
     return dq, dk, dv, None, None, None, None, None, None, None
 
@@ -576,7 +576,7 @@ def _backward_ex(ctx, grad_out, grad_lse, grad_ws):
                            "needs the log-sum-exp (windowed_attention sets it under autograd)")
     q, k, v, out, lse, mask, ws = ctx.saved_tensors
     mask_grad = mask is not None and mask.dtype != torch.bool and ctx.needs_input_grad[3]
-    op = _window_attn_bwd_ex if _lib.direct_call(grad_out, q, k, v) else window_attn_bwd_ex
+    op = _window_attn_bwd_ex if _lib.direct_backward(grad_out, q, k, v) else window_attn_bwd_ex
     dq, dk, dv, dm = op(grad_out, q, k, v, out, lse, mask, ws, *ctx.args, mask_grad)
     return (dq, dk, dv, dm if mask_grad else None, None, None, None, None, None, None, None, None,
             None)
@@ -704,12 +704,14 @@ class _FusedQKV(torch.autograd.Function):
         H, args, dropout_p, seed = ctx.call
         q, k, v = _split_heads(qkv, H)
         g = grad.reshape(out.shape)
-        if not _lib.direct_call(grad, qkv):  # a backward that is itself recorded: the registered ops
+        if not _lib.direct_backward(grad, qkv):  # recorded or batched: the registered ops
             if ws is None:
                 ds = window_attn_bwd(g, q, k, v, out, lse, *args)
             else:
                 ds = window_attn_bwd_ex(g, q, k, v, out, lse, mask, ws, *args, dropout_p, seed)[:3]
-            return torch.cat([d.transpose(1, 2).flatten(2) for d in ds], dim=-1), None, None, None, None, None
+            B, S = out.shape[:2]
+            return (torch.cat([d.transpose(1, 2).reshape(B, S, -1) for d in ds], dim=-1), None, None, None, None,
+                    None)
         B, S, _, dh = out.shape
         dqkv = torch.empty((B, S, 3, H, dh), dtype=qkv.dtype, device=qkv.device)
         grads = dqkv.unbind(2)
