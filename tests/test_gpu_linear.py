@@ -99,6 +99,19 @@ def test_projection_gradients_and_modes(dev):
     _close(y.detach().reshape(-1, 640), x.detach().reshape(-1, 192), q.weight.detach().bfloat16().t())
 
 
+@pytest.mark.gpu
+def test_result_changed_in_place(dev):
+    """A projection's result may be changed in place, as nn.Linear's: y += residual, in training."""
+    p = ln.Projection(192, 640).to(dev, torch.bfloat16)
+    x = torch.randn(10, 1201, 192, device=dev).bfloat16().requires_grad_()
+    gy = torch.randn(10, 1201, 640, device=dev).bfloat16()
+    want = torch.autograd.grad(p(x), [x, p.weight], gy)
+    y = p(x)
+    y += torch.ones_like(gy)
+    for a, b in zip(torch.autograd.grad(y, [x, p.weight], gy), want):
+        assert torch.equal(a, b)
+
+
 def test_projection_on_the_cpu_is_nn_linear():
     p = ln.Projection(64, 128)
     x = torch.randn(3, 5, 64, requires_grad=True)

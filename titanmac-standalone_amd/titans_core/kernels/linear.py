@@ -31,9 +31,11 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
     return t2
 
 
-def _fwd(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def _fwd(x2: torch.Tensor, w: torch.Tensor, lead=None) -> torch.Tensor:
+    """x2 [M, K] · wᵀ as [M, N], or [*lead, N]: not a view of it, which an autograd node may not return
+    to a caller that changes it in place."""
     (M, K), N = x2.shape, w.shape[0]
-    y = torch.empty((M, N), dtype=x2.dtype, device=x2.device)
+    y = torch.empty((M, N) if lead is None else (*lead, N), dtype=x2.dtype, device=x2.device)
     with _lib.device_guard(x2.device):
         rc = _lib.lib().tmac_linear_fwd(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                                         M, N, K, _lib.dtype_code(x2.dtype), _lib.stream_ptr(x2.device))
@@ -97,7 +99,7 @@ def _forward(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     N, K = weight.shape
     if not _fwd_applies(x.numel() // K, N, K):
         return F.linear(x, weight)
-    return _fwd(_rows(x), _rows(weight)).view(*x.shape[:-1], N)
+    return _fwd(_rows(x), _rows(weight), x.shape[:-1])
 
 
 class _Projection(torch.autograd.Function):
