@@ -112,6 +112,42 @@ def test_result_changed_in_place(dev):
         assert torch.equal(a, b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [3, 12010])
+@pytest.mark.parametrize("leaf_x", [False, True])
+def test_autocast_casts_the_weight_once(dev, rows, leaf_x):
+    """Eight calls in one autocast context keep one cast copy of the fp32 weight, as nn.Linear's do, both
+    where the kernels run and where the library does; the next context casts the changed weight again."""
+    p = ln.Projection(192, 640).to(dev)
+    x = torch.randn(rows, 192, device=dev).requires_grad_()
+    gy = torch.randn(rows, 640, device=dev)
+
+    def casts(fn):
+        kept = []
+        def pack(t):
+            if t.dtype == torch.bfloat16 and t.shape in (p.weight.shape, p.weight.t().shape):
+                kept.append(t)
+            return t
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t), torch.autocast("cuda", dtype=torch.bfloat16):
+            ys = [fn(x if leaf_x else x * (1 + 0 * i)) for i in range(8)]
+            assert all(y.dtype == torch.bfloat16 for y in ys)
+        (gw,) = torch.autograd.grad(sum(ys), p.weight, gy.bfloat16())
+        assert gw.dtype == torch.float32
+        return len({t.untyped_storage().data_ptr() for t in kept}), ys[0].detach(), gw
+    n, y, gw = casts(p)
+    n_ref, y_ref, gw_ref = casts(lambda t: F.linear(t, p.weight))
+    assert n == n_ref == 1
+    scale = gw_ref.abs().max()
+    assert torch.allclose(y.float(), y_ref.float(), rtol=2.0 ** -7, atol=2.0 ** -7)
+    assert torch.allclose(gw, gw_ref, rtol=2.0 ** -6, atol=2.0 ** -6 * scale)
+    with torch.no_grad():
+        p.weight.mul_(2)
+    _, y2, _ = casts(p)
+    assert torch.equal(y2, 2 * y)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(p(x), y2)
+
+
 def test_projection_on_the_cpu_is_nn_linear():
     p = ln.Projection(64, 128)
     x = torch.randn(3, 5, 64, requires_grad=True)

@@ -132,34 +132,49 @@ class _Projection(torch.autograd.Function):
         return gx, gw
 
 
+def _applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether a kernel takes a part of this call (of plain GPU tensors whose types it takes): by shape
+    alone, so that all other calls reach F.linear as they are."""
+    if weight.device != x.device or weight.dim() != 2 or x.dim() < 1 or x.shape[-1] != weight.shape[1] or x.numel() == 0:
+        return False
+    (N, K), M = weight.shape, x.numel() // x.shape[-1]
+    if N == 0 or N % 64 or K % 64 or max(N, K) > _MAX_PITCH or N * K > _MAX_WEIGHT or M > _MAX_ROWS:
+        return False
+    return _wgrad_applies(M) or _fwd_applies(M, N, K)
+
+
+def _autocast(t: torch.Tensor, dt: torch.dtype) -> torch.Tensor:
+    """t in the autocast type dt. A leaf that requires grad is cast through autocast's own cache, once per
+    autocast context, as for F.linear: a one-operand einsum returns the cast tensor itself."""
+    if t.dtype == dt or not (t.requires_grad and t.is_leaf):
+        return t.to(dt)
+    c = torch._VF.einsum("...->...", [t])
+    return c if c.dtype == dt else t.to(dt)
+
+
 def projection(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """F.linear(x, weight): [..., K] x [N, K] -> [..., N]. The kernels take bfloat16 and float16 (inside
     torch.autocast the inputs are cast to its dtype, as F.linear's are) with N and K multiples of 64."""
     ac = torch.is_autocast_enabled("cuda")
     if not (ac or x.dtype in _HALF) or not (x.is_cuda and weight.is_cuda and _lib.eager_native(x, weight)):
         return F.linear(x, weight)
+    grad = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
+    if not _applies(x, weight):
+        return F.linear(x, weight)
     if ac:
         dt = torch.get_autocast_dtype("cuda")
-        if dt in _HALF and x.dtype in (torch.float32, *_HALF) and weight.dtype in (torch.float32, *_HALF):
-            x, weight = x.to(dt), weight.to(dt)
-            with torch.autocast("cuda", enabled=False):
-                return _projection(x, weight)
+        if dt not in _HALF or not all(t.dtype in (torch.float32, *_HALF) for t in (x, weight)):
+            return F.linear(x, weight)
+        x, weight = _autocast(x, dt), _autocast(weight, dt)
+        with torch.autocast("cuda", enabled=False):
+            return _run(x, weight, grad)
+    if weight.dtype != x.dtype:
         return F.linear(x, weight)
-    return _projection(x, weight)
+    return _run(x, weight, grad)
 
 
-def _projection(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """projection outside autocast, of plain GPU tensors."""
-    if (x.dtype not in _HALF or weight.dtype != x.dtype or weight.device != x.device or weight.dim() != 2
-            or x.dim() < 1 or x.shape[-1] != weight.shape[1] or x.numel() == 0):
-        return F.linear(x, weight)
-    (N, K), M = weight.shape, x.numel() // x.shape[-1]
-    if (N == 0 or N % 64 or K % 64 or max(N, K) > _MAX_PITCH or N * K > _MAX_WEIGHT or M > _MAX_ROWS
-            or not (_wgrad_applies(M) or _fwd_applies(M, N, K))):
-        return F.linear(x, weight)
-    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
-        return _Projection.apply(x, weight)
-    return _forward(x, weight)
+def _run(x: torch.Tensor, weight: torch.Tensor, grad: bool) -> torch.Tensor:
+    return _Projection.apply(x, weight) if grad else _forward(x, weight)
 
 
 class Projection(nn.Linear):
