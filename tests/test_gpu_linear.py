@@ -148,6 +148,22 @@ def test_autocast_casts_the_weight_once(dev, rows, leaf_x):
         assert torch.equal(p(x), y2)
 
 
+def test_rules_stay_within_what_was_measured():
+    """(M, N, K) of each rule's edges: taken where the kernel measured faster, left to the library where it
+    measured slower (more than 5 %) or nothing was measured."""
+    for rule, taken, left in (
+            (ln._fwd_applies, [(17920, 1920, 640), (2240, 1920, 640), (17920, 640, 640), (12000, 768, 768), (32768, 384, 384)],
+             [(4480, 640, 640), (3000, 2304, 768), (17920, 768, 768), (6000, 2304, 768), (9000, 1536, 512), (9000, 1024, 1024)]),
+            (ln._dx_applies, [(17920, 1920, 640), (4480, 640, 640), (12000, 1536, 1536), (17920, 2048, 2048)],
+             [(9000, 1536, 1536), (17920, 2304, 768), (32768, 6144, 2048), (17920, 4096, 4096), (4480, 3072, 3072),
+              (32768, 3072, 1024), (12000, 1280, 1280)]),
+            (ln._wgrad_applies, [(17920, 1920, 640), (2240, 640, 640), (9000, 2048, 2048)],
+             [(512, 640, 640), (1100, 1024, 1024), (17920, 4608, 1536), (9000, 6144, 2048), (17920, 4096, 4096),
+              (4480, 12288, 4096), (1 << 20, 1 << 14, 1 << 14)])):
+        assert all(rule(*s) for s in taken), rule.__name__
+        assert not any(rule(*s) for s in left), rule.__name__
+
+
 def test_projection_on_the_cpu_is_nn_linear():
     p = ln.Projection(64, 128)
     x = torch.randn(3, 5, 64, requires_grad=True)

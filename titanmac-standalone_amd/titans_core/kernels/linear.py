@@ -68,31 +68,51 @@ def _wgrad(g2: torch.Tensor, x2: torch.Tensor) -> torch.Tensor:
     return dw
 
 
-# Where each kernel replaces the library's GEMM: where it measured faster (us, this kernel / library,
-# GPU time of [M, K] x [N, K] in bf16; `tiles` counts its 192 x 128 output tiles). A tile walks its
-# reduction in order, so few tiles or long walks leave the chip idle, and at K >= 1024 the library's
-# larger tiles read less through LDS.
+# Where each kernel replaces the library's GEMM: where it measured faster or as fast (us, this kernel /
+# library, GPU time of [M, K] x [N, K] in bf16; fp16 gives the same ratios to 9 %), over model widths 256 to
+# 4096, N = K and 3 K, and 512 to 32768 rows (of 315 sizes so taken, 9 are 3 to 7 % slower). Forward and dX walk 192 x 128 output tiles, two workgroups per CU: few
+# tiles, or a nearly empty last round of 512, leave the chip idle, and long walks and wide outputs are the
+# library's, whose larger tiles read less through LDS.
 
 def _tiles(rows: int, cols: int) -> int:
     return -(-rows // 192) * -(-cols // 128)
 
 
+def _fill(tiles: int) -> float:
+    """The share of the rounds of 512 workgroups that the tiles fill."""
+    return tiles / (512 * -(-tiles // 512))
+
+
 def _fwd_applies(M: int, N: int, K: int) -> bool:
-    """(2240, 640, 1920), 180 tiles: 12.1 / 15.0; (17920, 640, 1920): 54 / 80; (17920, 640, 640): 19 / 36;
-    below: (1100, 640, 1920), 90 tiles: 10.6 / 9.3; (9000, 1024, 3072): 60 / 51."""
-    return K <= 768 and _tiles(M, N) >= 150
+    """(17920, 640, 1920), as (M, K, N): 46 / 82; (17920, 640, 640): 18.5 / 35; (2240, 640, 1920), 180 tiles:
+    11.6 / 13.8; (12000, 768, 768), 378: 18.6 / 19.0; at K < 512 also rounds half empty: (32768, 384, 384),
+    fill 0.50: 18.9 / 24.9. Left to the library: (4480, 640, 640), 120 tiles: 10.8 / 8.7; (3000, 768, 2304),
+    288: 17.5 / 15.6; (17920, 768, 768), fill 0.55: 28.8 / 23.3; (4480, 1024, 3072): 34 / 26."""
+    if K > 768:
+        return False
+    t = _tiles(M, N)
+    return t >= (150 if K <= 512 else 180 if K <= 640 else 300) and (K < 512 or t <= 512 or _fill(t) >= 0.6)
 
 
 def _dx_applies(M: int, N: int, K: int) -> bool:
-    """(17920, 640, 1920), 470 tiles: 43 / 61; (9000, 1024, 3072), 376: 55 / 68; (4480, 640, 640), 120:
-    11.3 / 13.5; below: (4480, 640, 1920), 120: 26.2 / 25.2; (2240, 640, 640), 60: 10.7 / 8.4."""
-    return _tiles(M, K) >= (100 if N <= 1024 else 256)
+    """(17920, 640, 640): 18.5 / 38; (4480, 640, 640), 120 tiles: 11.2 / 13.2; (12000, 768, 768): 19.6 / 31;
+    (17920, 640, 1920), fill 0.92: 43 / 67; (12000, 1536, 1536), 0.74: 57 / 83. Left to the library:
+    (4480, 768, 768), 144 tiles: 12.9 / 12.2; (17920, 768, 768), fill 0.55: 31 / 27; (12000, 640, 1920), 0.62:
+    38 / 34; (9000, 1536, 1536), 0.55: 51 / 40; (32768, 1024, 3072): 196 / 165; (17920, 4096, 4096): 546 / 486."""
+    t = _tiles(M, K)
+    if N <= 640:
+        return t >= 100
+    if N <= 1024:
+        return t >= 180 and (t <= 512 or _fill(t) >= 0.6)
+    return N < 3072 and t <= 1536 and _fill(t) >= 0.7
 
 
-def _wgrad_applies(M: int) -> bool:
-    """The library gives these products few tiles and no split over M: (17920, 640, 1920): 59 / 141;
-    (17920, 640, 640): 28 / 102; (1100, 640, 640): 12.8 / 13.3; below: (256, 640, 640): 7.4 / 6.1."""
-    return M >= 512
+def _wgrad_applies(M: int, N: int, K: int) -> bool:
+    """The kernel splits the rows over the chip, which pays while the output has few tiles (of 256 x 128) and
+    the rows are many: (17920, 640, 1920): 63 / 145; (17920, 640, 640): 30 / 105; (2240, 640, 1920): 19.9 /
+    20.5; (17920, 2048, 2048), 128 tiles: 164 / 271. Left to the library: (1100, 1024, 1024): 14.8 / 13.2;
+    (512, 640, 640): 9.4 / 8.2; (17920, 1536, 4608), 216 tiles: 281 / 258; (4480, 3072, 3072): 131 / 92."""
+    return M >= 2048 and -(-N // 256) * -(-K // 128) <= 128
 
 
 def _forward(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -128,11 +148,11 @@ class _Projection(torch.autograd.Function):
             gx = gx.view(x.shape)
         if ctx.needs_input_grad[1]:
             x2 = x.reshape(-1, x.shape[-1])
-            gw = _wgrad(g2, _rows(x2)) if _wgrad_applies(M) else g2.t() @ x2
+            gw = _wgrad(g2, _rows(x2)) if _wgrad_applies(M, N, x2.shape[1]) else g2.t() @ x2
         return gx, gw
 
 
-def _applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
+def _applies(x: torch.Tensor, weight: torch.Tensor, grad: bool) -> bool:
     """Whether a kernel takes a part of this call (of plain GPU tensors whose types it takes): by shape
     alone, so that all other calls reach F.linear as they are."""
     if weight.device != x.device or weight.dim() != 2 or x.dim() < 1 or x.shape[-1] != weight.shape[1] or x.numel() == 0:
@@ -140,7 +160,7 @@ def _applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     (N, K), M = weight.shape, x.numel() // x.shape[-1]
     if N == 0 or N % 64 or K % 64 or max(N, K) > _MAX_PITCH or N * K > _MAX_WEIGHT or M > _MAX_ROWS:
         return False
-    return _wgrad_applies(M) or _fwd_applies(M, N, K)
+    return _fwd_applies(M, N, K) or grad and (_dx_applies(M, N, K) or _wgrad_applies(M, N, K))
 
 
 def _autocast(t: torch.Tensor, dt: torch.dtype) -> torch.Tensor:
@@ -159,7 +179,7 @@ def projection(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     if not (ac or x.dtype in _HALF) or not (x.is_cuda and weight.is_cuda and _lib.eager_native(x, weight)):
         return F.linear(x, weight)
     grad = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
-    if not _applies(x, weight):
+    if not _applies(x, weight, grad):
         return F.linear(x, weight)
     if ac:
         dt = torch.get_autocast_dtype("cuda")
