@@ -148,6 +148,35 @@ def test_autocast_casts_the_weight_once(dev, rows, leaf_x):
         assert torch.equal(p(x), y2)
 
 
+@pytest.mark.gpu
+def test_only_what_a_gradient_needs_is_kept(dev):
+    """As nn.Linear: with a frozen weight the input is not kept (and may change before the backward), for
+    an input without gradient the weight is not."""
+    p = ln.Projection(192, 640).to(dev, torch.bfloat16)
+    x = torch.randn(12010, 192, device=dev).bfloat16()
+    gy = torch.randn(12010, 640, device=dev).bfloat16()
+
+    def kept(x):
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t, lambda t: t):
+            y = p(x)
+        return y, seen
+    y, seen = kept(x)
+    assert seen == [x.shape]
+    with torch.no_grad():
+        p.weight.add_(1)
+    (gw,) = torch.autograd.grad(y, p.weight, gy)
+    _close(gw, gy.t(), x)
+    p.weight.requires_grad_(False)
+    leaf = x.clone().requires_grad_()
+    h = leaf * 1
+    y, seen = kept(h)
+    assert seen == [p.weight.shape]
+    h.add_(1)
+    (gx,) = torch.autograd.grad(y, leaf, gy)
+    _close(gx, gy, p.weight.detach())
+
+
 def test_rules_stay_within_what_was_measured():
     """(M, N, K) of each rule's edges: taken where the kernel measured faster, left to the library where it
     measured slower (more than 5 %) or nothing was measured."""

@@ -128,7 +128,9 @@ class _Projection(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight):
-        ctx.save_for_backward(x, weight)
+        # what a gradient needs, as nn.Linear keeps: frozen weights hold no activations, and the other
+        # operand may change before the backward
+        ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
         return _forward(x, weight)
 
     @staticmethod
@@ -145,7 +147,7 @@ class _Projection(torch.autograd.Function):
         M, N = g2.shape
         if ctx.needs_input_grad[0]:
             gx = _dx(g2, _rows(weight)) if _dx_applies(M, N, weight.shape[1]) else g2 @ weight
-            gx = gx.view(x.shape)
+            gx = gx.view(*gy.shape[:-1], weight.shape[1])
         if ctx.needs_input_grad[1]:
             x2 = x.reshape(-1, x.shape[-1])
             gw = _wgrad(g2, _rows(x2)) if _wgrad_applies(M, N, x2.shape[1]) else g2.t() @ x2
