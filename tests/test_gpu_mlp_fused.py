@@ -68,6 +68,24 @@ def test_fused_step_partial_gradients(dev):
 
 
 @pytest.mark.gpu
+def test_training_fc2_alone_keeps_no_pre_activation(dev):
+    """With fc1 frozen and an input without gradient, fc1 runs as in inference: nothing of it is kept."""
+    mlp = MLPBlock(128, 256, block_ell=True, density=0.5).to(dev, torch.bfloat16)
+    mlp.fc1.requires_grad_(False)
+    x, gy = (torch.randn(70, 128, device=dev).bfloat16() for _ in range(2))
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(tuple(t.shape)) or t, lambda t: t):
+        y = mlp(x)
+    assert sorted(seen) == sorted([(70, 256), tuple(mlp.fc2.values.shape), tuple(mlp.fc2.pattern.device_index(dev)["col_idx"].shape)])
+    y.backward(gy)
+    with torch.no_grad():
+        a = mlp.fc1(x, activation="gelu")
+        assert torch.equal(y, mlp.fc2(a))
+    want = kb._bell_sddmm(a, gy, mlp.fc2.pattern.device_index(dev)["col_idx"], *mlp.fc2.values.shape[:2], torch.bfloat16)
+    assert torch.equal(mlp.fc2.values.grad, want) and mlp.fc1.bias.grad is None
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("frozen", [(), ("fc1.values", "fc2.values", "x"), ("fc1.values", "fc1.bias", "fc2.values", "fc2.bias")])
 def test_second_derivatives_are_not_dropped(dev, frozen):
     """create_graph: the same first gradients, and what is built on them raises or is right (fc2's bias

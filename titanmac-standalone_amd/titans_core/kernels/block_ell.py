@@ -654,11 +654,12 @@ def _plain_layer(m: nn.Module) -> bool:
 
 def block_ell_mlp(x: torch.Tensor, fc1: "BlockELLLinear", fc2: "BlockELLLinear") -> torch.Tensor:
     """fc2(gelu(fc1(x))). A 16-bit training step of two plain layers is one autograd node (_MLP); every
-    other call runs the layers one after the other."""
+    other call runs the layers one after the other (also one that trains fc2 alone, where fc1 needs no
+    pre-activation)."""
     if (x.is_cuda and torch.is_grad_enabled() and _plain_layer(fc1) and _plain_layer(fc2) and x.numel() > 0
             and not torch.nn.modules.module._has_any_global_hook()):
         ts = (x, fc1.values, fc1.bias, fc2.values, fc2.bias)
-        if _lib.eager_native(*ts) and any(t is not None and t.requires_grad for t in ts):
+        if _lib.eager_native(*ts) and any(t is not None and t.requires_grad for t in ts[:3]):
             if torch.is_autocast_enabled("cuda"):
                 dt = torch.get_autocast_dtype("cuda")
                 if dt in (torch.bfloat16, torch.float16):
