@@ -51,16 +51,15 @@ def test_wgrad_split_over_rows(dev, M, N, K):
 
 @pytest.mark.gpu
 def test_rows_past_the_end_do_not_leak(dev):
-    """Infinities in the last row reach only what that row contributes to."""
+    """Infinities in the last row reach only what that row contributes to, and the last row counts once."""
     x = torch.ones(200, 64, device=dev, dtype=torch.bfloat16)
     x[-1] = float("inf")
     w = torch.ones(64, 64, device=dev, dtype=torch.bfloat16)
     y = ln._fwd(x, w)
     assert torch.all(y[:-1] == 64) and torch.all(torch.isinf(y[-1]))
     gy = torch.ones(200, 64, device=dev, dtype=torch.bfloat16)
-    gy[-1] = 0
-    x[-1] = 3
-    assert torch.all(ln._wgrad(gy, x) == 199)
+    x[-1] = 3  # the rows copied past the end repeat the last one: each would add 3
+    assert torch.all(ln._wgrad(gy, x) == 199 + 3)
 
 
 @pytest.mark.gpu

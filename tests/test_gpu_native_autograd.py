@@ -138,9 +138,10 @@ def test_eager_native_only_in_plain_eager_mode():
 @pytest.mark.parametrize("H,dh", [(2, 64), (3, 32), (1, 128), (2, 80)])
 @pytest.mark.parametrize("kw", [{}, {"pattern": "blockwin", "causal": False}, {"dropout_p": 0.2}, {"mask": "bool"},
                                 {"mask": "float"}])
-def test_fused_qkv_gradient(dev, dtype, H, dh, kw):
-    """The fused projection's gradient written in place equals the one autograd joins from q, k and v."""
-    from titans_core.kernels.window_attn import _split_heads, windowed_attention_qkv
+def test_fused_qkv_gradient(dev, dtype, H, dh, kw, monkeypatch):
+    """The fused projection's gradient written in place equals the one autograd joins from q, k and v
+    (head dimension 80, padded to 128, takes that general route itself)."""
+    from titans_core.kernels import window_attn as wa
     kw = dict(kw)
     g = torch.Generator().manual_seed(H * dh)
     B, S = 2, 150
@@ -148,18 +149,25 @@ def test_fused_qkv_gradient(dev, dtype, H, dh, kw):
     go = torch.randn(B, S, H * dh, generator=g).to(dev, dtype)
     mask = kw.pop("mask", None)
     if mask is not None:
-        mask = torch.rand(S, S, generator=g).to(dev)
-        mask = (mask > 0.4) | torch.eye(S, dtype=torch.bool, device=dev) if kw == {} and H == 2 else mask
+        keep = (torch.rand(S, S, generator=g) > 0.4) | torch.eye(S, dtype=torch.bool)
+        bias = torch.randn(S, S, generator=g).masked_fill(~keep, float("-inf"))
+        mask = {"bool": keep, "float": bias}[mask].to(dev)
     a, b = (qkv.clone().requires_grad_() for _ in range(2))
+    calls = []
+    fused = wa._FusedQKV.apply
+    monkeypatch.setattr(wa._FusedQKV, "apply", lambda *args: calls.append(1) or fused(*args))
     torch.manual_seed(7)
-    ya = windowed_attention_qkv(a, H, 40, 4, attn_mask=mask, **kw)
+    ya = wa.windowed_attention_qkv(a, H, 40, 4, attn_mask=mask, **kw)
+    assert len(calls) == (dh in wa.HEAD_DIMS)
     ya.backward(go)
     torch.manual_seed(7)
-    yb = windowed_attention(*_split_heads(b, H), 40, 4, attn_mask=mask, **kw).transpose(1, 2).reshape(B, S, -1)
+    yb = windowed_attention(*wa._split_heads(b, H), 40, 4, attn_mask=mask, **kw).transpose(1, 2).reshape(B, S, -1)
     yb.backward(go)
     assert torch.equal(ya, yb) and torch.equal(a.grad, b.grad)
+    assert torch.isfinite(a.grad).all()
     # an additive mask that needs its own gradient takes the general route
     if mask is not None and mask.is_floating_point():
         m = mask.clone().requires_grad_()
-        windowed_attention_qkv(a, H, 40, 4, attn_mask=m).backward(go)
-        assert m.grad is not None
+        del calls[:]
+        wa.windowed_attention_qkv(a, H, 40, 4, attn_mask=m).backward(go)
+        assert m.grad is not None and not calls
