@@ -1,6 +1,7 @@
 """dK/dV of the persistent keys at head dimension 64: their key block's list ends in a tail of query
-tiles that the waves share (one slice up to 32 persistent tokens, two up to 64, none past that). All
-gradients against the fp64 oracle, deterministic, at the edges of those ranges."""
+tiles that the waves share (one slice up to 32 persistent tokens, two up to 64, none past that, none in lists
+of less than 16 tiles or with a tail of less than 8). All gradients against the fp64 oracle, deterministic, at
+the edges of those ranges."""
 import numpy as np
 import pytest
 import torch
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dropout", [0.0, 0.2])
 @pytest.mark.parametrize("S,w,Np", [(900, 64, 1), (1300, 96, 16), (1301, 64, 32), (1100, 64, 33),
-                                    (1283, 100, 64), (1150, 64, 65), (576, 0, 5), (1217, 64, 128)])
+                                    (1283, 100, 64), (1150, 64, 65), (576, 0, 5), (1217, 64, 128),
+                                    (1000, 340, 16), (1000, 340, 48), (1000, 400, 16)])
 def test_persistent_key_tail(dev, S, w, Np, dropout):
     g = torch.Generator().manual_seed(S + Np)
     B, H, D = 1, 2, 64

@@ -23,7 +23,8 @@ pytestmark = pytest.mark.gpu
     (2, 521, 2048, 4),  # 8, 16
     (3, 1505, 2048, 4),  # 8, 32
     (3, 3009, 2048, 3),  # 16, 64
-    (40, 257, 512, 4),  # 8, 64: more than 512 partial rows of 16 or 32
+    (40, 257, 512, 4),  # 8, 32: more than 512 partial rows of 16
+    (40, 400, 512, 4),  # 8, 64: more than 512 partial rows of 32
     (2, 8001, 2048, 4),  # 32, 64
 ])
 def test_chunk_lengths(dev, dtype, B, T, C, k):
