@@ -907,9 +907,18 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void wattn_bwd_kv_kernel(
 constexpr int kKvStages = 4;
 constexpr int kKvTileB = 64 * 128;             // one 64x64 16-bit tile, bytes
 constexpr int kKvStageB = 2 * kKvTileB + 512;  // Q, dO, LSE·log2e, Δ
-constexpr int kKvTail = 8;  // entries from which a tail of one or two slices is shared by the waves
+// A tail is shared from kKvTail entries on, in lists of at least kKvList (whole backward, 16 persistent
+// tokens, 10 heads of 1000, window 64: 39.4 -> 30.9 us; a tail of 8, 10 heads of 1100, window 512: 49.5 ->
+// 44.5). From 4 entries in lists of 6 on, 10 heads of 600 measured 30.4 -> 26.8 and 80 heads of 400 with 48
+// persistent tokens 33.5 -> 35.1.
+constexpr int kKvTail = 8, kKvList = 16;
 
-template <int DT, int FEAT = 0>
+// SHARE: the waves may share the tail. Not with a caller's mask: the second copy of the tile's code costs
+// scalar registers and 5 % of the kernel there (45 -> 48 us on packed documents, 80 heads of 2000), and such
+// lists rarely have the tail. With dropout it spills 24 of them, which costs lists that have no tail 5 to 7
+// % of the backward (10 heads of 800, window 64: 53.4 -> 57.1 us), so there are two instances and
+// kv_has_tail chooses (10 heads of 4112: 203 -> 95 us). Without either it costs nothing: one instance.
+template <int DT, int FEAT = 0, bool SHARE = (FEAT & kFeatMask) == 0>
 __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     const uint16_t* __restrict__ dO, const float* __restrict__ lse, const float* __restrict__ delta,
@@ -921,9 +930,6 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     const int32_t* __restrict__ order, WorkMap wm, AttnX ax) {
   constexpr int D = 64;
   constexpr bool CM = (FEAT & kFeatMask) != 0, DR = (FEAT & kFeatDrop) != 0;
-  // With a caller's mask the second copy of the tile's code costs scalar registers and 5 % of the
-  // kernel (45 -> 48 us on packed documents, 80 heads of 2000), and such lists rarely have the tail.
-  constexpr bool kShare = !CM;
   using T = Tile<D>;
   __shared__ __attribute__((aligned(16))) uint16_t ring[kKvStages * kKvStageB / 2];
 
@@ -974,7 +980,7 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
   const int n = e1 - e0;
   // The list's tail in which only the first n_sl (1 or 2) key slices are listed, if it is long.
   int n_main = n, n_sl = 4;
-  if (kShare && n >= 16) {
+  if (SHARE && n >= kKvList) {
     int last1 = -1, last2 = -1;  // last entry listing a slice past the first, past the first two
     for (int base = 0; base < n; base += 64) {
       const int ent = base + lane < n ? entries[e0 + base + lane] : 0;
@@ -1139,7 +1145,7 @@ __global__ __launch_bounds__(256, 2) void wattn_bwd_kv64_kernel(
     process(ent, st, lse2);
     if constexpr (CM) wb = wb_next;
   }
-  if (kShare && n_main < n) {
+  if (SHARE && n_main < n) {
     // The tail: waves past the first n_sl write their finished slices, and wave w goes on with slice
     // w % n_sl, taking every (4 / n_sl)-th entry, copied whole into stage w, which is now its own.
     if (wave >= n_sl) {
@@ -2263,6 +2269,17 @@ void launch_fwd(const AttnLaunch& a) {
   }
 }
 
+// Whether the instance with dropout shares the persistent keys' tail: the query tiles past the last one that
+// sees key 127 (the span's end grows with the key), with the persistent keys in the first two of the block's
+// four slices. Where the grid fills the chip's 512 slots that one list sets the time only if most of it is
+// tail: 80 heads, window 512, 1100 rows (8 of 18 tiles) 120 -> 125 us, 2048 rows (22 of 32) 213 -> 206.
+bool kv_has_tail(const MaskParams& p, unsigned grid) {
+  const int n_t = (p.S + 63) / 64;
+  if (p.Np < 1 || p.Np > 64 || n_t < kKvList) return false;
+  const int tail = n_t - 1 - mask_col_span(p, 127).hi / 64;
+  return tail >= kKvTail && (grid <= 512 || 5 * tail >= 3 * n_t);
+}
+
 // Backward, 16-bit MFMA kernels: dQ (which also writes the row sums Δ), then dK/dV.
 template <int DT, int D, int FEAT>
 void launch_bwd_mfma(const AttnLaunch& a) {
@@ -2292,12 +2309,21 @@ void launch_bwd_mfma(const AttnLaunch& a) {
   // The copy-ring kernel addresses 64 rows of Q and dO with 32-bit byte offsets.
   if constexpr (D == 64) {
     if (qs[2] <= (1ll << 25) && gs[2] <= (1ll << 25)) {
-      hipLaunchKernelGGL((wattn_bwd_kv64_kernel<DT, (FEAT & ~kFeatDBias)>), dim3(a.grid_kv), dim3(256), 0, a.s, Q,
-                         K, V, G, a.lse, a.delta, static_cast<uint16_t*>(a.dK),
-                         static_cast<uint16_t*>(a.dV), qs[0], qs[1], qs[2], ks[0], ks[1], ks[2],
-                         vs[0], vs[1], vs[2], gs[0], gs[1], gs[2], dks[0], dks[1], dks[2], dvs[0],
-                         dvs[1], dvs[2], a.H, a.mp, a.scale, a.scale_log2, a.col_ptr,
-                         a.entries_kv, a.order_kv, a.wm_kv, a.ax_kv);
+      constexpr int F = FEAT & ~kFeatDBias;
+      constexpr bool kShared = (F & kFeatMask) == 0;
+#define TMAC_BWD_KV64(SHARE)                                                                          \
+  hipLaunchKernelGGL((wattn_bwd_kv64_kernel<DT, F, SHARE>), dim3(a.grid_kv), dim3(256), 0, a.s, Q, K, V, G, \
+                     a.lse, a.delta, static_cast<uint16_t*>(a.dK), static_cast<uint16_t*>(a.dV), qs[0], qs[1], \
+                     qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], gs[0], gs[1], gs[2], dks[0], dks[1], \
+                     dks[2], dvs[0], dvs[1], dvs[2], a.H, a.mp, a.scale, a.scale_log2, a.col_ptr,        \
+                     a.entries_kv, a.order_kv, a.wm_kv, a.ax_kv)
+      if constexpr (F == kFeatDrop) {
+        if (kv_has_tail(a.mp, a.grid_kv)) TMAC_BWD_KV64(true);
+        else TMAC_BWD_KV64(false);
+      } else {
+        TMAC_BWD_KV64(kShared);
+      }
+#undef TMAC_BWD_KV64
       return;
     }
   }
