@@ -1,4 +1,5 @@
-"""fp32 Block-ELL products at the edges of both tile heights (64 rows for small grids, 128 for large)."""
+"""fp32 Block-ELL products at the edges of both tile heights (64 rows for small grids, 128 for large ones and
+where long lists fill the CUs evenly)."""
 import pytest
 import torch
 
@@ -8,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,n_brow,n_bcol,width", [(1, 2, 3, 1), (63, 3, 5, 2), (64, 3, 5, 5), (65, 1, 4, 4), (127, 3, 2, 2),
-                                                   (129, 3, 5, 3), (6529, 3, 40, 10), (6528, 40, 3, 2)])
+                                                   (129, 3, 5, 3), (6529, 3, 40, 10), (6528, 40, 3, 2), (6401, 40, 10, 5),
+                                                   (4090, 16, 64, 32)])
 def test_f32_products(dev, M, n_brow, n_bcol, width):
     g = torch.Generator().manual_seed(M)
     pat = kb.BlockELLPattern.sample(2, n_brow, n_bcol, width)

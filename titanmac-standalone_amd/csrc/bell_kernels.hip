@@ -1488,8 +1488,16 @@ int launch_status() {
 // one (waves split its columns) gives twice the workgroups, four to a CU: below 2048 tiles of 128 rows
 // (eight per CU) the smaller one is faster: 2049 rows 640 -> 2560 at 50 %, 61 -> 56 us forward and 56 ->
 // 49 dX, 2560 -> 640 76 -> 63 and 45 -> 43, 500 rows 70 -> 39 us; at 8192 rows (2560 tiles) both take 153 us.
-int f32_rows(int M, int n_out) {
-  return static_cast<int64_t>((M + 127) / 128) * n_out < 2048 ? 64 : 128;
+// Between them, where long lists of 128-row tiles fill the CUs two or three deep almost evenly, the larger one
+// is (us, 64 / 128 rows): 9600 rows 2560 -> 640 at 50 % (750 tiles) 185 / 165, 8192 rows 3072 -> 768 (768)
+// 209 / 191, dX of 4096 rows 1024 -> 4096 (512) 161 / 151; 5000 rows (400) 109 / 114. Short or unequal lists
+// keep the smaller one: 640 -> 640 at 10 %, 6528 rows (510 tiles) 14.9 / 19.0. n_blocks: all the lists'
+// blocks, equal: lists of one length (dX).
+int f32_rows(int M, int n_out, int64_t n_blocks, bool equal) {
+  const int64_t t = static_cast<int64_t>((M + 127) / 128) * n_out;
+  if (t >= 2048) return 128;
+  const bool longl = equal ? n_blocks >= 8ll * n_out : n_blocks > 16ll * n_out;
+  return longl && ((t >= 400 && t <= 512) || (t >= 660 && t <= 768)) ? 128 : 64;
 }
 
 // Whether the SDDMM takes the rows' blocks four at a time across rows (NX = 2): with groups of one
@@ -1560,7 +1568,7 @@ int bell_fwd_impl(const void* d_X, int64_t ldx, const void* d_vals, const int32_
   if (d_bias && !aligned16(d_bias)) return TMAC_ERR_ALIGN;
   if (d_Z && (!aligned16(d_Z) || (ldz % vec))) return TMAC_ERR_ALIGN;
   if (dtype == TMAC_F32) {
-    const int bm = f32_rows(M, n_bcol), n_mt = (M + bm - 1) / bm;
+    const int bm = f32_rows(M, n_bcol, static_cast<int64_t>(n_brow) * width, false), n_mt = (M + bm - 1) / bm;
     const int64_t tot = static_cast<int64_t>(n_mt) * n_bcol;
     if (tot > (1ll << 30)) return TMAC_ERR_SHAPE;
     const int pxcd = static_cast<int>((tot + 7) / 8);
@@ -1732,7 +1740,7 @@ extern "C" int tmac_bell_dx(const void* d_dY, int64_t lddy, const void* d_vals,
   if (!aligned16(d_dY) || !aligned16(d_vals) || !aligned16(d_dX) || (lddy % vec) || (lddx % vec))
     return TMAC_ERR_ALIGN;
   if (dtype == TMAC_F32) {
-    const int bm = f32_rows(M, n_brow), n_mt = (M + bm - 1) / bm;
+    const int bm = f32_rows(M, n_brow, static_cast<int64_t>(n_brow) * width, true), n_mt = (M + bm - 1) / bm;
     const int64_t tot = static_cast<int64_t>(n_mt) * n_brow;
     if (tot > (1ll << 30)) return TMAC_ERR_SHAPE;
     const int pxcd = static_cast<int>((tot + 7) / 8);
