@@ -43,7 +43,20 @@ def test_f32_products(dev, M, n_brow, n_bcol, width):
 @pytest.mark.parametrize("n_brow,n_bcol,width", [(40, 10, 5), (7, 4, 3), (16, 8, 6), (9, 16, 9), (1, 8, 5)])
 @pytest.mark.parametrize("M", [1, 33, 700, 2100])
 def test_sddmm_blocks_across_rows(dev, M, n_brow, n_bcol, width, dtype):
-    """Widths whose blocks are taken four at a time across block-rows: every block of dW, twice the same."""
+    """Widths whose blocks fp32 takes four at a time across block-rows, from 256 rows on: every block of dW,
+    twice the same."""
+    _sddmm(dev, M, n_brow, n_bcol, width, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [8191, 8192, 8225])
+@pytest.mark.parametrize("n_brow", [31, 32, 41])
+def test_sddmm_blocks_across_rows_16_bit(dev, M, n_brow, dtype):
+    """The same in 16 bit: width 5, at least 40 groups (32 block-rows) and 8192 rows."""
+    _sddmm(dev, M, n_brow, 6, 5, dtype)
+
+
+def _sddmm(dev, M, n_brow, n_bcol, width, dtype):
     g = torch.Generator().manual_seed(M + width)
     pat = kb.BlockELLPattern.sample(3, n_brow, n_bcol, width)
     x = torch.randn(M, 64 * n_brow, generator=g).to(dev, dtype)

@@ -1200,7 +1200,12 @@ __global__ __launch_bounds__(256, BM == 64 ? 4 : 2) void bell_gemm_f32_kernel(
 // in LDS (rows past the range are zero); the wave's 64x64 block is four 32x32
 // MFMA tiles, an MFMA step summing rows m + 2s (lanes 0-31) and m + 2s + 1
 // (lanes 32-63). Partial sums go to the workspace as in the 16-bit kernel.
-template <int NX>
+constexpr int kSdChain = 128;  // rows summed in one chain of MFMAs
+
+// LONG: ranges of more than kSdChain rows, whose chains are added to running sums (64 more registers: two
+// waves per SIMD instead of four, 5 to 8 % of long ranges; a chain of a whole range took 1220 instead of 1320
+// us at 17920 x 4096 -> 4096, 25 %, with a relative error of 1.2e-6 instead of 2.4e-7).
+template <int NX, bool LONG>
 __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
     const float* __restrict__ X, int64_t ldx, const float* __restrict__ dY, int64_t lddy,
     const int32_t* __restrict__ col_idx, float* __restrict__ part, int M, int n_brow, int width,
@@ -1261,22 +1266,27 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       *reinterpret_cast<f32x4*>(ds[wave] + (4 * p + dr) * 64 + 4 * dc) = pd[p];
   };
 
-  // Sums of 128 rows, added to the running ones: short chains, so that a long range is summed as
+  // Sums of kSdChain rows, added to the running ones: short chains, so that a long range is summed as
   // exactly as many short ones.
-  f32x16 acc[2][2], tot[2][2];
+  f32x16 acc[2][2], run[LONG ? 2 : 1][LONG ? 2 : 1];
   auto flush = [&]() __attribute__((always_inline)) {
+    if constexpr (LONG) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        tot[a][b] += acc[a][b];
-        acc[a][b] = f32x16{};
-      }
+        for (int b = 0; b < 2; ++b) {
+          run[a][b] += acc[a][b];
+          acc[a][b] = f32x16{};
+        }
+    }
   };
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = tot[a][b] = f32x16{};
+    for (int b = 0; b < 2; ++b) {
+      acc[a][b] = f32x16{};
+      if constexpr (LONG) run[a][b] = f32x16{};
+    }
   if (m_lo < m_hi) gload(m_lo);
   for (int m = m_lo; m < m_hi; m += 32) {
     __syncthreads();
@@ -1295,7 +1305,7 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       acc[1][0] = mfma_f32(a1, b0, acc[1][0]);
       acc[1][1] = mfma_f32(a1, b1, acc[1][1]);
     }
-    if (((m - m_lo) & 96) == 96) flush();
+    if (((m - m_lo) & (kSdChain - 32)) == kSdChain - 32) flush();
   }
   flush();
 
@@ -1308,7 +1318,8 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int kk = 32 * a + 8 * (j >> 2) + 4 * h + (j & 3);
-        dst[kk * 64 + 32 * b + l32] = tot[a][b][j];
+        if constexpr (LONG) dst[kk * 64 + 32 * b + l32] = run[a][b][j];
+        else dst[kk * 64 + 32 * b + l32] = acc[a][b][j];
       }
 }
 
@@ -1502,32 +1513,41 @@ int f32_rows(int M, int n_out, int64_t n_blocks, bool equal) {
 
 // Whether the SDDMM takes the rows' blocks four at a time across rows (NX = 2): with groups of one
 // row's slots the last group of a width that is not a multiple of 4 has idle waves. The second X tile
-// makes a step's copies 24 KB instead of 20, so it pays where it saves more than a fifth of the
-// workgroups: widths 3, 5, 6, 9. Width 5, 2560 -> 640 at 50 %: bf16 32768 rows 92 -> 81 us, fp32 2049 rows 78 -> 56, 8192 rows 252 -> 172.
-bool sddmm_flat(int n_brow, int width) {
+// makes a step's copies 24 KB instead of 20, so in fp32 (bound by its MFMAs) it pays where it saves more
+// than a fifth of the workgroups, widths 3, 5, 6, 9: width 5, 2560 -> 640 at 50 %, 2049 rows 70 -> 51 us,
+// 8192 rows 223 -> 142, width 9 307 -> 261; below 256 rows it does not (12.3 against 11.9). In 16 bit (bound by
+// the copies) only width 5 saves enough, over many groups and rows: 2560 -> 640, 8192 rows 32.0 -> 30.5
+// us, 32768 rows 91 -> 81, but 4096 rows 22.2 -> 23.6; width 3 at 8192 rows 23.2 -> 26.4, width 6 21.7 -> 23.2.
+bool sddmm_flat(int M, int n_brow, int width, bool f32) {
+  if (width < 3) return false;
   const int64_t rows = static_cast<int64_t>(n_brow) * ((width + 3) / 4);
-  return width >= 3 && (static_cast<int64_t>(n_brow) * width + 3) / 4 * 6 < rows * 5;
+  const int64_t flat = (static_cast<int64_t>(n_brow) * width + 3) / 4;
+  return f32 ? M >= 256 && flat * 6 < rows * 5 : M >= 8192 && flat >= 40 && flat * 3 < rows * 2;
 }
-int sddmm_groups(int n_brow, int width) {
-  return sddmm_flat(n_brow, width) ? (n_brow * width + 3) / 4 : n_brow * ((width + 3) / 4);
+int sddmm_groups(int M, int n_brow, int width, bool f32) {
+  return sddmm_flat(M, n_brow, width, f32) ? (n_brow * width + 3) / 4 : n_brow * ((width + 3) / 4);
 }
 
 // Split of the SDDMM reduction over M, rows per split a multiple of 64: the cheapest of a model of its
-// time in microseconds. A CU that holds L workgroups takes a 64-row step of each in 0.7 L us (16 bit;
-// 1.05 alone) or 3.9 L + 0.3 (fp32, bound by its MFMAs; 5.2 alone); the partial sums are written and
-// read once at about 4.5 TB/s. (Filling 512 workgroup slots whatever M is wrote 8-11 partial copies of dW for a few
-// steps each: fp32 2049 x 640 -> 2560 55 -> 48 us, 2560 -> 640 56 -> 49, bf16 1000 x 640 -> 2560 22.5 -> 18.3.)
+// time in microseconds. A CU takes its L workgroups two at a time in 16 bit, a 64-row step of two in 1.4 us
+// and of one alone in 1.05; fp32 (bound by its MFMAs) takes a step of L in 3.9 L + 0.3 us (5.2 alone). The partial
+// sums are written and read once at about 4.5 TB/s, and the reduction of few blocks waits for each in turn.
+// (Filling 512 workgroup slots whatever M is wrote 8-11 partial copies of dW for a few steps each: fp32 2049 x
+// 640 -> 2560 55 -> 48 us, 2560 -> 640 56 -> 49, bf16 1000 x 640 -> 2560 22.5 -> 18.3. A CU's third workgroup priced
+// as a third of its load, and partial sums by their bytes alone, chose too many: bf16 32768 x 3072 -> 768 145
+// -> 121 us, fp32 4096 x 640 -> 640 at 10 % 38.7 -> 26.5.)
 void sddmm_split(int M, int n_brow, int width, bool f32, int* n_splits, int* rows_per_split) {
-  const int base = sddmm_groups(n_brow, width);
+  const int base = sddmm_groups(M, n_brow, width, f32);
   const int m_steps = (M + 63) / 64;
-  const float part_us = static_cast<float>(n_brow) * width * 16384.f * 2.f / 4.5e6f;
+  const float bytes_us = static_cast<float>(n_brow) * width * 16384.f * 2.f / 4.5e6f;
+  const float part_us = bytes_us > 0.35f ? bytes_us : 0.35f;
   float best_us = 0.f;
   const int most = 1024 / base > 1 ? 1024 / base : 1;  // up to four workgroups per CU
   for (int want = 1; want <= most && want <= m_steps; ++want) {
     const int steps = (m_steps + want - 1) / want;
     const int n = (m_steps + steps - 1) / steps;
     const int64_t load = (static_cast<int64_t>(n) * base + 255) / 256;
-    const float step_us = f32 ? (load == 1 ? 5.2f : 3.9f * load + 0.3f) : (load == 1 ? 1.05f : 0.7f * load);
+    const float step_us = f32 ? (load == 1 ? 5.2f : 3.9f * load + 0.3f) : 1.4f * (load / 2) + 1.05f * (load % 2);
     const float us = steps * step_us + n * part_us;
     if (want == 1 || us < best_us) {
       best_us = us;
@@ -1856,7 +1876,7 @@ extern "C" int tmac_bell_sddmm(const void* d_X, int64_t ldx, const void* d_dY, i
   // the 16-bit kernel addresses 32 rows of X and dY with 32-bit byte offsets
   if (dtype != TMAC_F32 && (ldx > (1ll << 25) || lddy > (1ll << 25))) return TMAC_ERR_SHAPE;
   const int n_sg = (width + 3) / 4;
-  const int64_t total = static_cast<int64_t>(n_splits) * sddmm_groups(n_brow, width);
+  const int64_t total = static_cast<int64_t>(n_splits) * sddmm_groups(M, n_brow, width, dtype == TMAC_F32);
   const int per_xcd = static_cast<int>((total + 7) / 8);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto* X = static_cast<const uint16_t*>(d_X);
@@ -1864,8 +1884,12 @@ extern "C" int tmac_bell_sddmm(const void* d_X, int64_t ldx, const void* d_dY, i
   float* part = static_cast<float*>(d_ws);
 #define TMAC_SDDMM_LAUNCH(NX)                                                                              \
   do {                                                                                                     \
-    if (dtype == TMAC_F32)                                                                                 \
-      hipLaunchKernelGGL(bell_sddmm_f32_kernel<NX>, dim3(8 * per_xcd), dim3(256), 0, s,                    \
+    if (dtype == TMAC_F32 && rows_per_split > kSdChain)                                                    \
+      hipLaunchKernelGGL((bell_sddmm_f32_kernel<NX, true>), dim3(8 * per_xcd), dim3(256), 0, s,            \
+                         static_cast<const float*>(d_X), ldx, static_cast<const float*>(d_dY), lddy,       \
+                         d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits, per_xcd);      \
+    else if (dtype == TMAC_F32)                                                                            \
+      hipLaunchKernelGGL((bell_sddmm_f32_kernel<NX, false>), dim3(8 * per_xcd), dim3(256), 0, s,           \
                          static_cast<const float*>(d_X), ldx, static_cast<const float*>(d_dY), lddy,       \
                          d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits, per_xcd);      \
     else if (dtype == TMAC_BF16)                                                                           \
@@ -1877,7 +1901,7 @@ extern "C" int tmac_bell_sddmm(const void* d_X, int64_t ldx, const void* d_dY, i
                          dY, lddy, d_col_idx, part, M, n_brow, width, n_sg, rows_per_split, n_splits,      \
                          per_xcd);                                                                         \
   } while (0)
-  if (sddmm_flat(n_brow, width))
+  if (sddmm_flat(M, n_brow, width, dtype == TMAC_F32))
     TMAC_SDDMM_LAUNCH(2);
   else
     TMAC_SDDMM_LAUNCH(1);
