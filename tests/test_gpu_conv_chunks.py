@@ -26,6 +26,8 @@ pytestmark = pytest.mark.gpu
     (40, 257, 512, 4),  # 8, 32: more than 512 partial rows of 16
     (40, 400, 512, 4),  # 8, 64: more than 512 partial rows of 32
     (2, 8001, 2048, 4),  # 32, 64
+    (17, 257, 512, 8),  # 16, 32: six taps and more in 16 bit, one round of 256 workgroups (fp32 16)
+    (40, 257, 512, 7),  # 16, 64 (fp32 32)
 ])
 def test_chunk_lengths(dev, dtype, B, T, C, k):
     g = torch.Generator().manual_seed(T + C + k)

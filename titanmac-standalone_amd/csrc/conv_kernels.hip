@@ -85,11 +85,15 @@ __device__ __forceinline__ void load_or_zero(const uint8_t* base, int64_t row_by
 // Forward / backward with the column sum, us, bf16, 1920 channels, 4 taps, 64-row chunks -> this rule:
 // 1 x 560 11.3 -> 3.5 / 25.3 -> 9.7, 8 x 560 13.7 -> 6.7 / 32.1 -> 20.8, 16 x 560 16.2 -> 12.8 / 34.4 ->
 // 27.0; 32 x 560 23.8 -> 22.8 / 43.1 (32 rows: 52.2); 8 x 4096 64 rows: 38.9 / 89.1 (32 rows: 39.5 / 94.6).
-// 600 partial rows: 32 x 600 x 768 backward 40.7 with 32 rows, 37.8 with 64. n: elements per 16-byte vector.
+// 600 partial rows: 32 x 600 x 768 backward 40.7 with 32 rows, 37.8 with 64. The 16-bit backward of six taps and
+// more takes 256 registers, one workgroup per CU, so a chunk is taken only while its workgroups make one
+// round: 8 taps, 12 x 560 x 1920 42 with 32 rows (216 workgroups), 67 with 64; 16 x 560 x 768 (288) 64 and
+// 58; 8 x 560 x 1920 16 rows (280) 46, 32 rows 40. n: elements per 16-byte vector.
 int conv_chunk(int B, int T, int C, int ks, int n, bool bwd) {
   for (int c = 8; c < 64; c *= 2) {
     const int64_t rows = static_cast<int64_t>(B) * ((T + c - 1) / c);
     const int64_t waves = (rows * (C / n) + 63) / 64;
+    if (bwd && n == 8 && ks >= 6 && rows * ((C / n + 255) / 256) > 256) continue;
     if (c >= 2 * (ks - 1) && waves <= (!bwd ? 2304 : c == 8 ? 512 : 1100) && (!bwd || rows <= 512)) return c;
   }
   return 64;
@@ -341,9 +345,10 @@ int launch_dwconv_bwd(const void* d_dout, int64_t ld_dout, const void* d_in, int
   return err == hipSuccess ? TMAC_OK : static_cast<int>(err);
 }
 
-// One size for every type: the 16-bit chunks are never longer than the fp32 ones.
+// One size for every type: that of the shorter chunk.
 size_t dwconv_bwd_ws_bytes(int B, int T, int C, int ks) {
-  const int chunk_len = conv_chunk(B, T, C, ks, 8, true);
+  const int c16 = conv_chunk(B, T, C, ks, 8, true), c32 = conv_chunk(B, T, C, ks, 4, true);
+  const int chunk_len = c16 < c32 ? c16 : c32;
   const int64_t n_chunks = (T + chunk_len - 1) / chunk_len;
   return static_cast<size_t>(B) * n_chunks * C * ks * sizeof(float);
 }
