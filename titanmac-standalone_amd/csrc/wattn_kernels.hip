@@ -1958,58 +1958,62 @@ __global__ __launch_bounds__(256) void wattn_mask_kinds_kernel(AttnX ax, int S, 
   uint64_t row0 = 0, row1 = 0;    // lane r < 32: allowed bits of row r, key tiles 2j, 2j + 1
   const int k0 = j * 128 + lane, k1 = k0 + 64;
   // The loads of kB rows are in flight before their ballots (with a test of the format and the edges
-  // around each load they stood one latency after another): bool masks 16 rows, 15.6 -> 10.3 us at S =
-  // 1537 and 22.3 -> 16.6 at 4096; float masks, four times the bytes, 8 rows (16 rows cost occupancy:
-  // 21.4 -> 24.0 at 4096, now 22.8). Positions past S read the last row or key and count as masked.
+  // around each load they stood one latency after another), and the groups of rows are a loop (unrolled
+  // whole, the rows' addresses spilled 140 scalar registers): all three launches, bool masks, 16 rows, 20.6 -> 11.4
+  // us at S = 1537 and 26.2 -> 18.0 at 4096; float masks, four times the bytes, 8 rows, 14.9 -> 11.8 and 24.9 ->
+  // 23.1 (16 rows 25.4, 4 rows 22.6, but 18.5 for four masks of 1537, 8 rows 17.7). Positions past S read the last
+  // row or key and count as masked.
   constexpr int kB = BOOL ? 16 : 8;
   const int64_t moff = (ax.mb1 ? 0 : static_cast<int64_t>(bm) * ax.msb) +
                        (ax.mh1 ? 0 : static_cast<int64_t>(hm) * ax.msh);
   const int q0 = i * 128 + 32 * wave;
   const int kc0 = min(k0, S - 1), kc1 = min(k1, S - 1);
-  float v[2][kB];
+#pragma unroll 1
+  for (int rb = 0; rb < 32; rb += kB) {
+    float v[2][kB];
+    if constexpr (BOOL) {
+      const uint8_t* m = static_cast<const uint8_t*>(ax.mask) + moff;
+      uint8_t t[2][kB];
 #pragma unroll
-  for (int r = 0; r < 32; ++r) {
-    if (r % kB == 0) {
-      if constexpr (BOOL) {
-        const uint8_t* m = static_cast<const uint8_t*>(ax.mask) + moff;
-        uint8_t t[2][kB];
+      for (int rr = 0; rr < kB; ++rr) {
+        const uint8_t* row = m + static_cast<int64_t>(min(q0 + rb + rr, S - 1)) * ax.msq;
+        t[0][rr] = row[kc0];
+        t[1][rr] = row[kc1];
+      }
 #pragma unroll
-        for (int rr = 0; rr < kB; ++rr) {
-          const uint8_t* row = m + static_cast<int64_t>(min(q0 + r + rr, S - 1)) * ax.msq;
-          t[0][rr] = row[kc0];
-          t[1][rr] = row[kc1];
-        }
+      for (int rr = 0; rr < kB; ++rr) {
+        v[0][rr] = t[0][rr] ? 0.f : -INFINITY;
+        v[1][rr] = t[1][rr] ? 0.f : -INFINITY;
+      }
+    } else {
+      const float* m = static_cast<const float*>(ax.mask) + moff;
 #pragma unroll
-        for (int rr = 0; rr < kB; ++rr) {
-          v[0][rr] = t[0][rr] ? 0.f : -INFINITY;
-          v[1][rr] = t[1][rr] ? 0.f : -INFINITY;
-        }
-      } else {
-        const float* m = static_cast<const float*>(ax.mask) + moff;
-#pragma unroll
-        for (int rr = 0; rr < kB; ++rr) {
-          const float* row = m + static_cast<int64_t>(min(q0 + r + rr, S - 1)) * ax.msq;
-          v[0][rr] = row[kc0];
-          v[1][rr] = row[kc1];
-        }
+      for (int rr = 0; rr < kB; ++rr) {
+        const float* row = m + static_cast<int64_t>(min(q0 + rb + rr, S - 1)) * ax.msq;
+        v[0][rr] = row[kc0];
+        v[1][rr] = row[kc1];
       }
     }
-    const bool in = q0 + r < S;
-    const float v0 = in && k0 < S ? v[0][r % kB] : -INFINITY;
-    const float v1 = in && k1 < S ? v[1][r % kB] : -INFINITY;
-    const bool a0 = !(v0 == -INFINITY), a1 = !(v1 == -INFINITY);
-    any0 |= a0;
-    all0 &= (v0 == 0.f);
-    nz0 |= a0 & (v0 != 0.f);
-    any1 |= a1;
-    all1 &= (v1 == 0.f);
-    nz1 |= a1 & (v1 != 0.f);
-    col0 |= static_cast<uint32_t>(a0) << r;
-    col1 |= static_cast<uint32_t>(a1) << r;
-    const uint64_t w0 = __ballot(a0), w1 = __ballot(a1);
-    if (lane == r) {
-      row0 = w0;
-      row1 = w1;
+#pragma unroll
+    for (int rr = 0; rr < kB; ++rr) {
+      const int r = rb + rr;
+      const bool in = q0 + r < S;
+      const float v0 = in && k0 < S ? v[0][rr] : -INFINITY;
+      const float v1 = in && k1 < S ? v[1][rr] : -INFINITY;
+      const bool a0 = !(v0 == -INFINITY), a1 = !(v1 == -INFINITY);
+      any0 |= a0;
+      all0 &= (v0 == 0.f);
+      nz0 |= a0 & (v0 != 0.f);
+      any1 |= a1;
+      all1 &= (v1 == 0.f);
+      nz1 |= a1 & (v1 != 0.f);
+      col0 |= static_cast<uint32_t>(a0) << r;
+      col1 |= static_cast<uint32_t>(a1) << r;
+      const uint64_t w0 = __ballot(a0), w1 = __ballot(a1);
+      if (lane == r) {
+        row0 = w0;
+        row1 = w1;
+      }
     }
   }
   // bitmaps
