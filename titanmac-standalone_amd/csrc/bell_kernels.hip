@@ -1202,16 +1202,19 @@ __global__ __launch_bounds__(256, BM == 64 ? 4 : 2) void bell_gemm_f32_kernel(
 // (lanes 32-63). Partial sums go to the workspace as in the 16-bit kernel.
 constexpr int kSdChain = 128;  // rows summed in one chain of MFMAs
 
-// LONG: ranges of more than kSdChain rows, whose chains are added to running sums (64 more registers: two
-// waves per SIMD instead of four, 5 to 8 % of long ranges; a chain of a whole range took 1220 instead of 1320
-// us at 17920 x 4096 -> 4096, 25 %, with a relative error of 1.2e-6 instead of 2.4e-7).
+// LONG: ranges of more than kSdChain rows, whose chains are added to running sums. Those take 64 more
+// registers, two workgroups per CU instead of four, which leaves room for two stages (NX = 1): the next tile
+// is stored while this one's math goes on, with one barrier per tile. 17920 x 4096 -> 4096 at 25 %: a chain of the
+// whole range 1224 us with a relative error of 1.2e-6, running sums 1326 and with two stages 1276 us with 2.4e-7;
+// 8192 x 512 -> 2048 at 50 % 88, 92 and 88 us.
 template <int NX, bool LONG>
 __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
     const float* __restrict__ X, int64_t ldx, const float* __restrict__ dY, int64_t lddy,
     const int32_t* __restrict__ col_idx, float* __restrict__ part, int M, int n_brow, int width,
     int n_sgroups, int rows_per_split, int n_splits, int per_xcd) {
-  __shared__ __attribute__((aligned(16))) float xs[NX][32 * 64];
-  __shared__ __attribute__((aligned(16))) float ds[4][32 * 64];
+  constexpr int kSt = LONG && NX == 1 ? 2 : 1;  // stages: two fit where two workgroups share a CU
+  __shared__ __attribute__((aligned(16))) float xs[kSt][NX][32 * 64];
+  __shared__ __attribute__((aligned(16))) float ds[kSt][4][32 * 64];
 
   const int n_blocks = n_brow * width;
   const int per_split = NX == 1 ? n_brow * n_sgroups : (n_blocks + 3) / 4;
@@ -1256,14 +1259,14 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       pd[p] = *reinterpret_cast<const f32x4*>(dY + static_cast<int64_t>(row) * lddy + 64 * c + 4 * dc);
     }
   };
-  auto sstore = [&]() __attribute__((always_inline)) {
+  auto sstore = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
-      for (int x = 0; x < NX; ++x) *reinterpret_cast<f32x4*>(xs[x] + (16 * p + xr) * 64 + 4 * xc) = px[x][p];
+      for (int x = 0; x < NX; ++x) *reinterpret_cast<f32x4*>(xs[b][x] + (16 * p + xr) * 64 + 4 * xc) = px[x][p];
 #pragma unroll
     for (int p = 0; p < 8; ++p)
-      *reinterpret_cast<f32x4*>(ds[wave] + (4 * p + dr) * 64 + 4 * dc) = pd[p];
+      *reinterpret_cast<f32x4*>(ds[b][wave] + (4 * p + dr) * 64 + 4 * dc) = pd[p];
   };
 
   // Sums of kSdChain rows, added to the running ones: short chains, so that a long range is summed as
@@ -1287,16 +1290,12 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       acc[a][b] = f32x16{};
       if constexpr (LONG) run[a][b] = f32x16{};
     }
-  if (m_lo < m_hi) gload(m_lo);
-  for (int m = m_lo; m < m_hi; m += 32) {
-    __syncthreads();
-    sstore();
-    __syncthreads();
-    if (m + 32 < m_hi) gload(m + 32);
-    const float* dsw = ds[wave];
-    const float* xsw = xs[xt_own];
+  // rows 16 half..+15 of stage b
+  auto math = [&](int b, int half) __attribute__((always_inline)) {
+    const float* dsw = ds[b][wave];
+    const float* xsw = xs[b][xt_own];
 #pragma unroll
-    for (int st = 0; st < 16; ++st) {
+    for (int st = 8 * half; st < 8 * half + 8; ++st) {
       const int row = 2 * st + h;
       const float a0 = xsw[row * 64 + l32], a1 = xsw[row * 64 + 32 + l32];
       const float b0 = dsw[row * 64 + l32], b1 = dsw[row * 64 + 32 + l32];
@@ -1305,7 +1304,37 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       acc[1][0] = mfma_f32(a1, b0, acc[1][0]);
       acc[1][1] = mfma_f32(a1, b1, acc[1][1]);
     }
-    if (((m - m_lo) & (kSdChain - 32)) == kSdChain - 32) flush();
+  };
+  if (m_lo < m_hi) {
+    gload(m_lo);
+    if constexpr (kSt == 2) {
+      sstore(0);
+      if (m_lo + 32 < m_hi) gload(m_lo + 32);
+      __syncthreads();
+    }
+  }
+  for (int m = m_lo; m < m_hi; m += 32) {
+    if constexpr (kSt == 2) {
+      // the next tile into the other stage (read last before the barrier that ended the last step) while
+      // this one's math goes on
+      const int b = ((m - m_lo) >> 5) & 1;
+      math(b, 0);
+      if (m + 32 < m_hi) {
+        sstore(b ^ 1);
+        if (m + 64 < m_hi) gload(m + 64);
+      }
+      math(b, 1);
+      if (((m - m_lo) & (kSdChain - 32)) == kSdChain - 32) flush();
+      __syncthreads();
+    } else {
+      __syncthreads();
+      sstore(0);
+      __syncthreads();
+      if (m + 32 < m_hi) gload(m + 32);
+      math(0, 0);
+      math(0, 1);
+      if (((m - m_lo) & (kSdChain - 32)) == kSdChain - 32) flush();
+    }
   }
   flush();
 
