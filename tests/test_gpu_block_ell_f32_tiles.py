@@ -71,3 +71,17 @@ def _sddmm(dev, M, n_brow, n_bcol, width, dtype):
     # fp32 sums of exact products in any order (16-bit) or of rounded ones (fp32)
     err = (dv.double() - blocks(x, gy)).abs()
     assert torch.all(err <= (M + 2) * 2.0 ** -24 * blocks(x.abs(), gy.abs()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [40, 700])
+@pytest.mark.parametrize("width", [2, 5])
+def test_sddmm_infinity_in_the_last_row(dev, M, width, dtype):
+    """An infinite gradient in the last row gives infinities of the right sign: rows past the range add nothing."""
+    pat = kb.BlockELLPattern.sample(1, 3, 6, width)
+    x = torch.ones(M, 192, device=dev, dtype=dtype)
+    x[-1, ::2] = -1
+    gy = torch.ones(M, 384, device=dev, dtype=dtype)
+    gy[-1] = float("inf")
+    dv = kb._bell_sddmm(x, gy, torch.from_numpy(pat.col_idx).to(dev).reshape(-1), 3, width, torch.float32)
+    assert torch.all(dv[:, :, ::2] == float("-inf")) and torch.all(dv[:, :, 1::2] == float("inf"))

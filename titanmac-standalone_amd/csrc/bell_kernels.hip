@@ -1259,7 +1259,12 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       pd[p] = *reinterpret_cast<const f32x4*>(dY + static_cast<int64_t>(row) * lddy + 64 * c + 4 * dc);
     }
   };
-  auto sstore = [&](int b) __attribute__((always_inline)) {
+  auto sstore = [&](int b, int m) __attribute__((always_inline)) {
+    if (m + 32 > m_hi) {  // both factors are zero past the range: 0 times an infinity of the last row is none
+#pragma unroll
+      for (int p = 0; p < 8; ++p)
+        if (m + 4 * p + dr >= m_hi) pd[p] = f32x4{};
+    }
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
@@ -1308,7 +1313,7 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
   if (m_lo < m_hi) {
     gload(m_lo);
     if constexpr (kSt == 2) {
-      sstore(0);
+      sstore(0, m_lo);
       if (m_lo + 32 < m_hi) gload(m_lo + 32);
       __syncthreads();
     }
@@ -1320,7 +1325,7 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       const int b = ((m - m_lo) >> 5) & 1;
       math(b, 0);
       if (m + 32 < m_hi) {
-        sstore(b ^ 1);
+        sstore(b ^ 1, m + 32);
         if (m + 64 < m_hi) gload(m + 64);
       }
       math(b, 1);
@@ -1328,7 +1333,7 @@ __global__ __launch_bounds__(256, 2) void bell_sddmm_f32_kernel(
       __syncthreads();
     } else {
       __syncthreads();
-      sstore(0);
+      sstore(0, m);
       __syncthreads();
       if (m + 32 < m_hi) gload(m + 32);
       math(0, 0);
