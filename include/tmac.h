@@ -547,7 +547,7 @@ int tmac_dwconv_causal_bwd_workspace(int B, int T, int C, int ksize, size_t* ws_
  * :234-236). d_out, in, d_in: [B, T, C] with row strides ld_dout, ld_in,
  * ld_din, same dtype and alignment rules as tmac_dwconv_causal; w: [C, ksize]
  * in that dtype; dw: fp32 [C, ksize], overwritten (not accumulated). The
- * weight gradient is summed per 64-position chunk into the workspace, then
+ * weight gradient is summed per chunk of 8 to 64 positions into the workspace, then
  * over the chunks in a fixed order, so it is deterministic. */
 int tmac_dwconv_causal_bwd(const void* d_dout, int64_t ld_dout, const void* d_in,
                            int64_t ld_in, const void* d_w, void* d_din, int64_t ld_din,
